@@ -24,7 +24,8 @@ static_assert(SH_dtbeta_z == SH_dtbeta_r + 1, "dtbeta_r and dtbeta_z planes are 
 enum ScalarSlot { SC_phi = 0, SC_xi_r, SC_xi_z, SC_pi, NSCALAR };
 
 // Planes of the per-level buffer of geometric auxiliaries that the first
-// phase of the RHS kernel writes and the second reads: the Ricci tensor (A,
+// phase of the two-phase RHS kernel writes, for its second phase and for the
+// constraints: the Ricci tensor (A,
 // B, C components and the scalar) and the divergences DIV_KT, DIVA_KT.
 enum AuxSlot {
   AUX_RA = 0, AUX_RB, AUX_RC, AUX_RSCAL, AUX_DIV_r, AUX_DIV_z, AUX_DIVA_r, AUX_DIVA_z, NAUX
@@ -46,6 +47,19 @@ struct KGrid {
   double dr, dz, dt;
   double idr, idz;      // 1/dr, 1/dz
   double zoff;          // z_j = (j - zoff) * dz
+};
+
+// Stencil weights of a level, formed on the host so that they reach the
+// kernel in scalar registers: the 1/dr, 1/12, ... factors of the centred
+// stencils folded together, the dissipation strengths, and the upwinded
+// derivative split into its odd and even parts (advdis in oaxis_rhs.h).
+struct KStencil {
+  double r12, z12;      // 1/(12 dr), 1/(12 dz)
+  double rr12, zz12;    // 1/(12 dr^2), 1/(12 dz^2)
+  double rz3, rz48;     // 1/(3 dr dz), 1/(48 dr dz)
+  double ar[3], az[3];  // advection of the geometry: weights of f(+k) - f(-k), k = 1, 2, 3
+  double ur, uz;        // and of |beta| D6 (0 with centred advection)
+  double ko_g, ko_s;    // KO weight of the geometry and of the scalar field
 };
 
 // Physics switches and constants of one right-hand-side launch.
@@ -95,8 +109,12 @@ size_t fb_record_bytes();                     // sizeof(FbPoint)
 // grid.  A spacetime alone launches tables of one item; a batch of
 // spacetimes launches one table over all its members.
 struct RhsItem {                  // one RK substep of a level
-  KGrid G; KPhys P; KStep S;
+  KGrid G; KPhys P; KStep S; KStencil W;
   const double* yin; const double* yp; double* acc; double* yout; double* gaux;
+  // the computed points: i in [1, ihi], j in [jlo, jhi]; with skip, those of
+  // the frame around i <= sihi, j in [sjlo, sjhi] alone
+  int ihi, jlo, jhi;
+  int skip, sihi, sjlo, sjhi;
   int nbi, nbj;                   // 16 x 16 tiles along r and z
   int block0;
 };
@@ -134,9 +152,17 @@ int del_blocks(const DelItem& it);
 int save_blocks(const SaveItem& it);
 int fb_blocks(const FbItem& it, bool shift, bool scalar);
 int rs_blocks(const RsItem& it);
-// tiles of a level for the RHS kernel; OA_ERR_ARG if a direction has fewer
-// than 16 points
-int rhs_tiles(const KGrid& G, int* nbi, int* nbj);
+// The computed points and tiles of a level for the RHS kernel; OA_ERR_ARG if
+// a direction has fewer than 16 points.  inner: without the outer 3 rows,
+// which finebound fills after every substep of a fine level.  Where the rest
+// would have fewer than 16 points in a direction the whole level is taken
+// (*inner set to false).
+int rhs_tiles(RhsItem* it, bool* inner);
+// the frame left out by it, an item with inner tiles: the same substep on
+// the outer rows alone
+RhsItem rhs_frame(const RhsItem& it);
+// stencil weights of a level
+void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W);
 
 // raise the LDS limits of the RHS kernels (once, before any launch)
 int prepare_rhs_kernels();

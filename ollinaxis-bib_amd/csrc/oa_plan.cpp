@@ -309,8 +309,8 @@ int plan_level(Plan& plan, const std::vector<oa_handle*>& all, int level) {
       substep_weights(h, level, iter, &dtw, &w);
       dtws[k] = dtw;
       RhsItem it;
-      bool pm = false;
-      RC(prepare_substep(h, level, iter, ni, dtw, w, &it, &pm));
+      bool pm = false, inner = false;
+      RC(prepare_substep(h, level, iter, ni, dtw, w, &it, &pm, &inner));
       rhs[group_code(h->shift, h->scalar) * 2 + (pm ? 1 : 0)].push_back(it);
     }
     for (int c = 0; c < 8; ++c) plan.add(K_RHS, (c & 4) != 0, (c & 2) != 0, (c & 1) != 0, rhs[c]);

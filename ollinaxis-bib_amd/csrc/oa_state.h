@@ -78,8 +78,10 @@ namespace oax {
 int niter_of(const oa_handle* h);
 void substep_weights(const oa_handle* h, int level, int iter, double* dtw, double* w);
 int prepare_saveold(oa_handle* h, int level, SaveItem* it);
+// *inner: the item leaves out the outer rows that finebound fills (rhs_frame
+// gives them)
 int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, double w, RhsItem* it,
-                    bool* phimode);
+                    bool* phimode, bool* inner);
 bool prepare_finebound(oa_handle* h, int level, double dtw, FbItem* it);   // false on level 0
 // auxiliary(level): *proj / *del say whether the projection / DelDef run
 void prepare_auxiliary(oa_handle* h, int level, ProjItem* pj, bool* proj, DelItem* dd, bool* del);

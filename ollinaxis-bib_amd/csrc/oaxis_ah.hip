@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) k_ah_fields(KGrid G, const double* __rest
   const int j = G.jlo + static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   const int i = 1 + static_cast<int>(blockIdx.y * blockDim.y + threadIdx.y);
   if (j > G.Nz || i > G.Nr) return;
-  const GlobalView V{y, G, nullptr};
+  const GlobalView V{y, G};
   const double r = (static_cast<double>(i) - 0.5) * G.dr;
   const double chi = V.fld(S_chi)(i, j);
   const double phi = phi_from_chi ? -std::log(chi) / 2.0 : V.fld(S_phi)(i, j);

@@ -255,20 +255,26 @@ struct Proj {
   double chi, phi, A, B, H, C;
 };
 
-OA_HD void project(Proj& q, double r, bool time0, int chimethod, bool matter) {
+OA_HD void project_factor(Proj& q, bool time0, int chimethod, bool matter) {
   if (!chimethod || time0) {
     q.chi = exp(-2.0 * q.phi);
     if (chimethod && matter) q.phi = -0.5 * log(q.chi);
   } else {
     q.phi = -0.5 * log(q.chi);
   }
-  if (!time0) {
-    const double rc = r * q.C;
-    double aux = (q.A * q.B - rc * rc) * q.H;
-    aux = cbrt(aux);
-    const double ia = 1.0 / aux;
-    q.A *= ia; q.B *= ia; q.C *= ia; q.H *= ia;
-  }
+}
+
+OA_HD void factordet(Proj& q, double r) {
+  const double rc = r * q.C;
+  double aux = (q.A * q.B - rc * rc) * q.H;
+  aux = cbrt(aux);
+  const double ia = 1.0 / aux;
+  q.A *= ia; q.B *= ia; q.C *= ia; q.H *= ia;
+}
+
+OA_HD void project(Proj& q, double r, bool time0, int chimethod, bool matter) {
+  project_factor(q, time0, chimethod, matter);
+  if (!time0) factordet(q, r);
 }
 
 // write v at (i,j) and, inside the symmetry bands, its parity images
@@ -302,7 +308,12 @@ OA_HD void slot_parity(bool shift, bool scalar, int s, double& symr, double& sym
 // never formed (they keep their initial zero).  This holds for the first step
 // of a level and for the first internal iteration of its second step.
 // S.proj_t0: the auxiliary call that ends this iteration runs at clock 0.
-template <bool SHIFT, bool SCALAR, bool PHIMODE, bool IN, int STAGE, class View>
+//
+// In two phases, one thread per point: the Gamma-driver in vacuum
+// (k_rhs_phases), and phase 1 alone for the constraints.  The other
+// configurations take rhs_roles (oaxis_rhs.h), which sums the same terms in
+// another order.
+template <bool SHIFT, bool PHIMODE, bool IN, int STAGE, class View>
 OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View& V,
                      const double* __restrict__ yp, double* __restrict__ acc, double* __restrict__ yout,
                      double* __restrict__ gaux, int i, int j) {
@@ -428,11 +439,11 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
   const double Dra = da.r, Dza = da.z, Drp = dp.r, Dzp = dp.z;
 
   // ---- geometric auxiliaries: D_i D_j alpha, the Ricci tensor, div KT.
-  // STAGE 0 computes them in place, STAGE 1 computes the Ricci tensor and
-  // div KT and stores them (one plane each in gaux, AUX_* order) and returns,
-  // STAGE 2 reads them back.  D_i D_j alpha and its trace are formed where
-  // they are used (STAGE 0 and 2) from the lapse and metric derivatives that
-  // phase holds anyway, rather than passed through gaux.
+  // STAGE 1 computes the Ricci tensor and div KT and stores them (one plane
+  // each in gaux, AUX_* order) and returns, STAGE 2 reads them back.  D_i D_j
+  // alpha and its trace are formed where they are used (STAGE 2) from the
+  // lapse and metric derivatives that phase holds anyway, rather than passed
+  // through gaux.
   double d2A, d2B, d2C, Lapla, RA, RB, RC, RSCAL, DIV_r, DIV_z, DIVA_r, DIVA_z;
   auto lapse_hessian = [&]() {
     // D_i D_j alpha and its trace (:1268-1324)
@@ -461,8 +472,7 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
     DIV_r = ax[AUX_DIV_r * pl]; DIV_z = ax[AUX_DIV_z * pl]; DIVA_r = ax[AUX_DIVA_r * pl]; DIVA_z = ax[AUX_DIVA_z * pl];
     lapse_hessian();
   } else {
-    if constexpr (STAGE != 12) {
-      if constexpr (STAGE == 0) lapse_hessian();
+    {
 
       // ---- Ricci tensor (:1397-1493 and calc_conformalRicci1..4, non-angmom)
       double RH;
@@ -545,7 +555,7 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
       RSCAL = (gA * RA + gB * RB + gH * RH + 2.0 * r2 * gC * RC) * ipsi4;
 
     }
-    if constexpr (STAGE != 11) {
+    {
       // ---- divergence of KT (calc_DIVKTA.f90:573-636)
       {
         const double Ar = dA.r, Az = dA.z, Br = dB.r, Bz = dB.z, Hr = dH.r, Hz = dH.z, Cr = dC.r, Cz = dC.z;
@@ -599,96 +609,13 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
       }
     }
   }
-  // STAGE 11 / 12: the two halves of STAGE 1 (the Ricci tensor; div KT),
-  // for kernels that run them one after the other
-  if constexpr (STAGE == 1 || STAGE == 11 || STAGE == 12) {
+  if constexpr (STAGE == 1) {
     double* const ax = gaux + k;
-    if constexpr (STAGE != 12) {
-      ax[AUX_RA * pl] = RA; ax[AUX_RB * pl] = RB; ax[AUX_RC * pl] = RC; ax[AUX_RSCAL * pl] = RSCAL;
-    }
-    if constexpr (STAGE != 11) {
-      ax[AUX_DIV_r * pl] = DIV_r; ax[AUX_DIV_z * pl] = DIV_z; ax[AUX_DIVA_r * pl] = DIVA_r; ax[AUX_DIVA_z * pl] = DIVA_z;
-    }
+    ax[AUX_RA * pl] = RA; ax[AUX_RB * pl] = RB; ax[AUX_RC * pl] = RC; ax[AUX_RSCAL * pl] = RSCAL;
+    ax[AUX_DIV_r * pl] = DIV_r; ax[AUX_DIV_z * pl] = DIV_z; ax[AUX_DIVA_r * pl] = DIVA_r; ax[AUX_DIVA_z * pl] = DIVA_z;
     return;
   }
 
-
-  // ---- real scalar field: auxiliary_matter / potential / stressenergy
-  double rho = 0.0, J_r = 0.0, J_z = 0.0, mS_A = 0.0, mS_B = 0.0, mS_H = 0.0, mS_C = 0.0, trS = 0.0;
-  double s_sphi = 0.0, s_sxr = 0.0, s_sxz = 0.0, s_spi = 0.0;
-  double sc_phi = 0.0, sc_xr = 0.0, sc_xz = 0.0, sc_pi = 0.0;
-  constexpr double smallpi = 3.14159265358979323846;
-  const double dscale_s = P.scalardiss / G.dt;
-  if constexpr (SCALAR) {
-    const auto Fsp = fld(scalar_slot(SHIFT, SC_phi)), Fxr = fld(scalar_slot(SHIFT, SC_xi_r));
-    const auto Fxz = fld(scalar_slot(SHIFT, SC_xi_z)), Fpi = fld(scalar_slot(SHIFT, SC_pi));
-    sc_phi = Fsp(i, j); sc_xr = Fxr(i, j); sc_xz = Fxz(i, j); sc_pi = Fpi(i, j);
-    double V = 0.0, VP = 0.0;
-    if (P.scalarpotential == OA_POT_PHI2) {
-      V = 0.5 * P.scalar_mass * P.scalar_mass * sc_phi * sc_phi;
-      VP = P.scalar_mass * P.scalar_mass * sc_phi;
-    } else if (P.scalarpotential == OA_POT_PHI4) {
-      V = 0.5 * P.scalar_mass * P.scalar_mass * sc_phi * sc_phi + 0.25 * P.scalar_lambda * sc_phi * sc_phi * sc_phi * sc_phi;
-      VP = P.scalar_mass * P.scalar_mass * sc_phi + P.scalar_lambda * sc_phi * sc_phi * sc_phi;
-    }
-    const double xr = sc_xr, xz = sc_xz, pi = sc_pi;
-    const double q2 = (gA * xr * xr + gB * xz * xz + 2.0 * r * gC * xr * xz) * ipsi4;
-    rho = 0.5 * (pi * pi + q2) + V;
-    J_r = -(gA * xr + r * gC * xz) * pi * ipsi4;
-    J_z = -(gB * xz + r * gC * xr) * pi * ipsi4;
-    const double aux = 0.5 * (pi * pi - q2) - V;
-    const double psi4 = 1.0 / ipsi4;
-    mS_A = xr * xr + A * psi4 * aux;
-    mS_B = xz * xz + B * psi4 * aux;
-    mS_C = xr * xz * ir + C * psi4 * aux;
-    mS_H = H * psi4 * aux;
-    trS = (gA * mS_A + gB * mS_B + gH * mS_H + 2.0 * r2 * gC * mS_C) * ipsi4;
-
-    // sources_scalar (scalar.f90:94-251)
-    const D1 dpi = grad<IN>(Fpi, G, i, j);
-    s_sphi = alpha * pi;
-    if constexpr (SHIFT) s_sphi += br * xr + bz * xz;
-    s_sxr = alpha * dpi.r + pi * Dra;
-    s_sxz = alpha * dpi.z + pi * Dza;
-    if constexpr (SHIFT) {
-      const D1 dxr = grad<IN>(Fxr, G, i, j), dxz = grad<IN>(Fxz, G, i, j);
-      s_sxr += br * s_adr<IN>(Fxr, G, i, j, br) + xr * dbr_.r + bz * s_adz<IN>(Fxr, G, i, j, bz) + xz * dbz_.r;
-      s_sxz += br * s_adr<IN>(Fxz, G, i, j, br) + xr * dbr_.z + bz * s_adz<IN>(Fxz, G, i, j, bz) + xz * dbz_.z;
-      (void)dxr; (void)dxz;
-    }
-    double dr_, dz_, lap;
-    if (P.scalarmethod == OA_SCALARMETHOD_FIRST) {
-      const D1 dxr = grad<IN>(Fxr, G, i, j), dxz = grad<IN>(Fxz, G, i, j);
-      dr_ = xr; dz_ = xz;
-      lap = alpha * (gA * dxr.r + gB * dxz.z + r * gC * (dxz.r + dxr.z));
-    } else {
-      const D2 ds = hess<IN>(Fsp, G, i, j);
-      dr_ = ds.r; dz_ = ds.z;
-      lap = alpha * (gA * ds.rr + gB * ds.zz + 2.0 * r * gC * ds.rz);
-    }
-    double spi = lap;
-    spi += 2.0 * alpha * (Drp * (gA * dr_ + r * gC * dz_) + Dzp * (gB * dz_ + r * gC * dr_));
-    spi += Dra * (gA * dr_ + r * gC * dz_) + Dza * (gB * dz_ + r * gC * dr_);
-    spi += alpha * (dr_ * (dgA.r + r * dgC.z) + dz_ * (dgB.z + r * dgC.r + gC));
-    spi += alpha * (gA * dr_ * ir + gC * dz_);
-    spi = spi * ipsi4;
-    spi += alpha * pi * trK;
-    if (P.scalarpotential != OA_POT_NONE) spi -= alpha * VP;
-    if constexpr (SHIFT) spi += br * s_adr<IN>(Fpi, G, i, j, br) + bz * s_adz<IN>(Fpi, G, i, j, bz);
-    if (P.scalardiss != 0.0) {
-      s_sphi -= s_ko<IN>(Fsp, G, i, j, dscale_s);
-      spi -= s_ko<IN>(Fpi, G, i, j, dscale_s);
-      s_sxr -= s_ko<IN>(Fxr, G, i, j, dscale_s);
-      s_sxz -= s_ko<IN>(Fxz, G, i, j, dscale_s);
-    }
-    // radiative boundary on pi at every level (scalar.f90:244-251)
-    const bool bnd = (i == G.Nr) || (j == G.Nz) || (!G.eqsym && j == 1 - G.g);
-    if (!IN && bnd) {
-      const double rr = sqrt(r * r + z * z);
-      spi = -(r * dpi.r + z * dpi.z + pi) / rr;
-    }
-    s_spi = spi;
-  }
 
   // ---- sources_geometry (sources_geometry.f90:77-575), lagrangian: sigma = 1
   const double dscale_g = P.geodiss / G.dt;
@@ -723,7 +650,6 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
       adv(FK, dK, DAr, DAz);
       strK += br * DAr + bz * DAz;
     }
-    if constexpr (SCALAR) strK += 4.0 * smallpi * alpha * (rho + trS);
     if (P.geodiss != 0.0) strK -= s_ko<IN>(FK, G, i, j, dscale_g);
   }
 
@@ -742,13 +668,6 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
     adv(FKC, dKC, DAr, DAz);
     sKTC += br * DAr + bz * DAz + KTC * br * ir + KTC * (dbr_.r + dbz_.z) + (KTB * dbz_.r + KTA * dbr_.z) * ir
             - t23 * KTC * DIV_beta;
-  }
-  if constexpr (SCALAR) {
-    const double psi4 = 1.0 / ipsi4;
-    (void)psi4;
-    sKTA -= 8.0 * smallpi * alpha * (mS_A * ipsi4 - third * A * trS);
-    sKTB -= 8.0 * smallpi * alpha * (mS_B * ipsi4 - third * B * trS);
-    sKTC -= 8.0 * smallpi * alpha * (mS_C * ipsi4 - third * C * trS);
   }
   if (P.geodiss != 0.0) {
     sKTA -= s_ko<IN>(FKA, G, i, j, dscale_g);
@@ -772,11 +691,6 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
     sDz += br * DAr + bz * DAz - Delta_r * dbz_.r - Delta_z * dbz_.z;
     sDz += 2.0 * r * gC * dbz_.rz + gA * dbz_.rr + gB * dbz_.zz + gH * dbz_.r * ir;
     sDz += third * (r * gC * Dr_DIV_beta + gB * Dz_DIV_beta + 2.0 * Delta_z * DIV_beta);
-  }
-  if constexpr (SCALAR) {
-    const double psi4 = 1.0 / ipsi4;
-    sDr -= 8.0 * smallpi * eta * alpha * J_r * psi4;
-    sDz -= 8.0 * smallpi * eta * alpha * J_z * psi4;
   }
   if (P.geodiss != 0.0) {
     sDr -= s_ko<IN>(FDr, G, i, j, dscale_g);
@@ -861,7 +775,7 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
   // y_p and the accumulator of every slot, loaded together before any store
   // (so one memory round trip serves them all); on the first iteration the
   // staged input is y_p itself
-  constexpr int NF = nslots(SHIFT, SCALAR);
+  constexpr int NF = nslots(SHIFT, false);
   double yv[NF], av[NF];
 #pragma unroll
   for (int q = 0; q < NF; ++q) yv[q] = yp[q * pl + k];
@@ -903,7 +817,7 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
     Dr_n = rk(S_Delta_r, sDr);
     Dz_n = rk(S_Delta_z, sDz);
   }
-  project(q, r, pt0, P.chimethod, SCALAR);
+  project(q, r, pt0, P.chimethod, false);
 
   double* const yo = yout;
   put(yo + S_alpha * pl, G, i, j, alpha_n, 1.0, 1.0);
@@ -926,12 +840,6 @@ OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View&
     put(yo + shift_slot(SH_beta_z) * pl, G, i, j, rk(shift_slot(SH_beta_z), sbz), 1.0, -1.0);
     put(yo + shift_slot(SH_dtbeta_r) * pl, G, i, j, rk(shift_slot(SH_dtbeta_r), sdbr), -1.0, 1.0);
     put(yo + shift_slot(SH_dtbeta_z) * pl, G, i, j, rk(shift_slot(SH_dtbeta_z), sdbz), 1.0, -1.0);
-  }
-  if constexpr (SCALAR) {
-    put(yo + scalar_slot(SHIFT, SC_phi) * pl, G, i, j, rk(scalar_slot(SHIFT, SC_phi), s_sphi), 1.0, 1.0);
-    put(yo + scalar_slot(SHIFT, SC_xi_r) * pl, G, i, j, rk(scalar_slot(SHIFT, SC_xi_r), s_sxr), -1.0, 1.0);
-    put(yo + scalar_slot(SHIFT, SC_xi_z) * pl, G, i, j, rk(scalar_slot(SHIFT, SC_xi_z), s_sxz), 1.0, -1.0);
-    put(yo + scalar_slot(SHIFT, SC_pi) * pl, G, i, j, rk(scalar_slot(SHIFT, SC_pi), s_spi), 1.0, 1.0);
   }
 }
 

@@ -162,7 +162,7 @@ int prepare_saveold(oa_handle* h, int level, SaveItem* it) {
 }
 
 int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, double w, RhsItem* it,
-                    bool* phimode) {
+                    bool* phimode, bool* inner) {
   Level& L = h->L[level];
   if (!L.in_step) {
     oa_set_error("oa_substep called before oa_saveold");
@@ -173,7 +173,12 @@ int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, do
     return OA_ERR_STATE;
   }
   *it = RhsItem{};
-  RC(rhs_tiles(L.G, &it->nbi, &it->nbj));
+  it->G = L.G;
+  // finebound, which follows every substep of a fine level, fills at least
+  // its outer ghost-width rows, and nothing reads them (or their accumulator)
+  // in between: the substep computes the points inside them
+  *inner = level > 0;
+  RC(rhs_tiles(it, inner));
   const int a = L.step_a;
   const int in = (iter == 1) ? a : L.last_out;
   int out;
@@ -185,11 +190,11 @@ int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, do
   }
   const bool time0 = (L.t == 0.0);
   *phimode = L.aux_phi;
-  it->G = L.G;
   it->P = h->phys;
   it->P.radiative = (level == 0 && h->p.boundtype == OA_BOUND_RADIATIVE) ? 1 : 0;
   it->S = KStep{iter, niter, h->p.integrator == OA_RK4 ? 1 : 0, dtw, w, time0 ? 1 : 0,
                 L.dtb_pre_valid ? L.dtb_pre : nullptr};
+  rhs_stencil(it->G, it->P, &it->W);
   it->yin = L.slab[in];
   it->yp = L.slab[a];
   it->acc = L.acc;
@@ -328,10 +333,13 @@ int do_saveold(oa_handle* h, int level) {
 
 int do_substep(oa_handle* h, int level, int iter, int niter, double dtw, double w) {
   RhsItem it;
-  bool phimode = false;
-  RC(prepare_substep(h, level, iter, niter, dtw, w, &it, &phimode));
+  bool phimode = false, inner = false;
+  RC(prepare_substep(h, level, iter, niter, dtw, w, &it, &phimode, &inner));
   h->plan.begin();
-  h->plan.add_one(K_RHS, h->shift, h->scalar, phimode, it);
+  // on its own a substep leaves every point advanced: the outer rows too
+  std::vector<RhsItem> items(1, it);
+  if (inner) items.push_back(rhs_frame(it));
+  h->plan.add(K_RHS, h->shift, h->scalar, phimode, items);
   return h->plan.submit(h->stream);
 }
 

@@ -25,6 +25,7 @@
 #define OA_HD __device__ __forceinline__
 #define OA_HHD __host__ __device__ inline
 #include "oaxis_device.h"
+#include "oaxis_rhs.h"
 
 namespace oax {
 
@@ -35,17 +36,19 @@ namespace oax {
   } while (0)
 
 // ------------------------------------------------------------ RHS kernel
-// Each 16 x 16 block stages its tile of every field, with a 3-point halo, in
+// Each block stages a 16 x 16 tile of every field, with a 3-point halo, in
 // LDS and reads all stencils from there.  Centred stencils reach 3 points.
 // The one-sided closures at i = Nr-1..Nr, j = Nz-1..Nz and (without
 // equatorial symmetry) j = 1-ghost..2-ghost reach up to 5 points, always
 // towards the interior; the first and the last tile of each direction are
-// anchored to the ends of the level, so those reads stay inside the tile.
-// The last tile of a direction may overlap the one before it; its points
-// already covered there are skipped (the RK accumulator is read-modify-write).
+// anchored to the ends of the computed range, so those reads stay inside the
+// tile.  The last tile of a direction may overlap the one before it; its
+// points already covered there are skipped (the RK accumulator is
+// read-modify-write).
 constexpr int kTile = 16, kHalo = 3;
 constexpr int kTileW = kTile + 2 * kHalo;                 // staged extent per direction
 constexpr int kTileSize = kTileW * kTileW;                // values per field
+constexpr int kRhsBlock = 512;                            // two waves per 64 points
 
 // first point of tile b of nb along [lo, hi] (extent >= kTile)
 __host__ __device__ inline int tile_start(int b, int nb, int lo, int hi) {
@@ -58,31 +61,15 @@ __device__ __forceinline__ bool interior_tile(const KGrid& G, int i0, int j0) {
   return i0 >= 1 && i0 + kTile - 1 <= G.Nr - 3 && j0 >= 1 && j0 + kTile - 1 <= G.Nz - 3;
 }
 
-// Staging an RHS input tile into LDS.  Each thread owns the same two points
-// of every staged plane, q0 = tid and q1 = tid + 256 (the tile has 484), so
-// their offsets in a plane are worked out once.  Points of the tile outside
-// the level, which no stencil reads, take the value of the nearest point
-// inside it, so that every load is in bounds and none needs a branch.
-struct StageSlots {
-  long o0, o1;          // plane offsets of the two points
-  int q0, q1;           // their tile positions
-  bool two;             // q1 lies inside the tile
-};
-
-__device__ __forceinline__ StageSlots stage_slots(const KGrid& G, int ib, int jb) {
-  StageSlots s;
-  const int tid = static_cast<int>(threadIdx.y) * kTile + static_cast<int>(threadIdx.x);
+// Staging an RHS input tile into LDS: each of the first 484 threads owns one
+// point of every staged plane, so its offset in a plane is worked out once.
+// Points of the tile outside the level, which no stencil reads, take the
+// value of the nearest point inside it, so that every load is in bounds and
+// none needs a branch.
+__device__ __forceinline__ long stage_offset(const KGrid& G, int ib, int jb, int q) {
   const int lo = 1 - G.g;
-  s.q0 = tid;
-  s.q1 = tid + kTile * kTile;
-  s.two = s.q1 < kTileSize;
-  auto offset = [&](int q) {
-    const int ii = min(max(ib + q / kTileW, lo), G.Nr), jj = min(max(jb + q % kTileW, lo), G.Nz);
-    return IDX(G, ii, jj);
-  };
-  s.o0 = offset(s.q0);
-  s.o1 = s.two ? offset(s.q1) : s.o0;
-  return s;
+  const int ii = min(max(ib + q / kTileW, lo), G.Nr), jj = min(max(jb + q % kTileW, lo), G.Nz);
+  return IDX(G, ii, jj);
 }
 
 // Stage NST planes, plane f from src(f), into tile slots first .. first +
@@ -90,20 +77,12 @@ __device__ __forceinline__ StageSlots stage_slots(const KGrid& G, int ib, int jb
 // their latencies overlap instead of adding up (a load-wait-store loop per
 // plane waits out one memory round trip per plane and point).
 template <int NST, class Src>
-__device__ __forceinline__ void stage_planes(double* tile, int first, const StageSlots& s, Src src) {
-  double v0[NST], v1[NST];
+__device__ __forceinline__ void stage_planes(double* tile, int first, int q, long off, Src src) {
+  double v[NST];
 #pragma unroll
-  for (int f = 0; f < NST; ++f) {
-    const double* __restrict__ p = src(f);
-    v0[f] = p[s.o0];
-    v1[f] = p[s.o1];
-  }
+  for (int f = 0; f < NST; ++f) v[f] = src(f)[off];
 #pragma unroll
-  for (int f = 0; f < NST; ++f) {
-    double* dst = tile + (first + f) * kTileSize;
-    dst[s.q0] = v0[f];
-    if (s.two) dst[s.q1] = v1[f];
-  }
+  for (int f = 0; f < NST; ++f) tile[(first + f) * kTileSize + q] = v[f];
 }
 
 // Pointers read from a work item are generic; every one of them addresses
@@ -144,22 +123,20 @@ __device__ __forceinline__ const Item& find_item(const Item* __restrict__ items,
   return items[lo];
 }
 
-// One RK substep of a level: each 16 x 16 block stages its tile and runs two
-// phases per point.  Phase 1 forms the geometric auxiliaries (the Ricci
-// tensor and div KT: the longest expressions, which need only the vacuum
-// fields) and passes them through the per-level buffer gaux; phase 2 forms
-// D_i D_j alpha, every source, the dissipation, the radiative boundaries and
-// the RK update.  Kept apart, the phases need at most the registers of the
-// larger one.
-// Occupancy of the RHS kernel.  With the Gamma-driver or the scalar field the
-// staged tile (17 or 21 fields, 66-81 KB) allows two blocks per CU, and the
-// two phases fit 256 VGPRs: two waves per SIMD.  In vacuum the tile (13
-// fields, 50 KB) allows three blocks, and phase 1 split in two halves fits
-// 168 VGPRs: three waves per SIMD.
+// the 1/r column table of a tile, in LDS after its planes
+__device__ __forceinline__ void stage_inv_r(const KGrid& G, double* rinv, int ib, int q) {
+  if (q < kTileW) rinv[q] = 1.0 / ((static_cast<double>(ib + q) - 0.5) * G.dr);
+}
+
+// One RK substep of a level.  A block stages its tile once and eight waves
+// work on it: waves 0-3 form one half of the sources of the tile's points,
+// waves 4-7 the other half (rhs_roles), so the LDS of a tile serves twice the
+// waves that one thread per point would give.  The halves are about equal in
+// instructions per point.
 template <bool SHIFT, bool SCALAR>
-constexpr bool kSplitPhase1 = !SHIFT && !SCALAR;
+constexpr int kRole0 = ROLE_K | (SHIFT && SCALAR ? ROLE_SCALAR : SHIFT || SCALAR ? ROLE_LAPSE : 0);
 template <bool SHIFT, bool SCALAR>
-constexpr int kRhsBlocksPerCu = kSplitPhase1<SHIFT, SCALAR> ? 3 : 2;
+constexpr int kRole1 = (ROLE_DELTA | ROLE_LAPSE | ROLE_METRIC | ROLE_SCALAR) & ~kRole0<SHIFT, SCALAR>;
 
 template <bool SHIFT, bool SCALAR, bool PHIMODE>
 __device__ __forceinline__ void rhs_tile(const RhsItem& it, int bi, int bj, double* tile) {
@@ -168,46 +145,42 @@ __device__ __forceinline__ void rhs_tile(const RhsItem& it, int bi, int bj, doub
   KStep S = it.S;
   S.dtb_pre = gmem(S.dtb_pre);            // null stays null
   const int nbj = it.nbj, nbi = it.nbi;
-  const int j0 = tile_start(bj, nbj, G.jlo, G.Nz);
-  const int i0 = tile_start(bi, nbi, 1, G.Nr);
+  const int j0 = tile_start(bj, nbj, it.jlo, it.jhi);
+  const int i0 = tile_start(bi, nbi, 1, it.ihi);
   const int ib = i0 - kHalo, jb = j0 - kHalo;
-  // the evolved fields, then (first substep only) the dtbeta planes it differentiates
+  if (it.skip && i0 + kTile - 1 <= it.sihi && j0 >= it.sjlo && j0 + kTile - 1 <= it.sjhi) return;
+  const int tid = static_cast<int>(threadIdx.x);
+  // the evolved fields, then (first substep only) the dtbeta planes it
+  // differentiates, then the 1/r table
   const double* __restrict__ yin = gmem(it.yin);
-  double* const gaux = gmem(it.gaux);
-  {
-    const StageSlots ss = stage_slots(G, ib, jb);
-    stage_planes<nf>(tile, 0, ss, [&](int f) { return yin + f * G.plane; });
-    if (S.dtb_pre) stage_planes<2>(tile, nf, ss, [&](int f) { return S.dtb_pre + f * G.plane; });
-    __syncthreads();
+  double* const rinv = tile + (nf + (SHIFT && S.dtb_pre ? 2 : 0)) * kTileSize;
+  if (tid < kTileSize) {
+    const long off = stage_offset(G, ib, jb, tid);
+    stage_planes<nf>(tile, 0, tid, off, [&](int f) { return yin + f * G.plane; });
+    if (SHIFT && S.dtb_pre) stage_planes<2>(tile, nf, tid, off, [&](int f) { return S.dtb_pre + f * G.plane; });
   }
-  const int i = i0 + static_cast<int>(threadIdx.y), j = j0 + static_cast<int>(threadIdx.x);
+  stage_inv_r(G, rinv, ib, tid);
+  __syncthreads();
+  const int p = tid & 255;
+  const int di = p / kTile, dj = p % kTile;
+  const int i = i0 + di, j = j0 + dj;
   if (bi == nbi - 1 && i < 1 + (nbi - 1) * kTile) return;        // done by the tile before
-  if (bj == nbj - 1 && j < G.jlo + (nbj - 1) * kTile) return;
-  const TileView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, nf};
-  // phase 1: the geometric auxiliaries of this point, through gaux (own point
-  // only, so no synchronisation); the memory barrier keeps the compiler from
-  // carrying phase-1 values or loads into phase 2, so the two phases do not
-  // add up in registers
-  if constexpr (kSplitPhase1<SHIFT, SCALAR>) {
-    // vacuum: phase 1 in its two halves (the Ricci tensor, then div KT),
-    // so that no part needs more than 168 VGPRs: three waves per SIMD
-    if (interior_tile(G, i0, j0)) {
-      rhs_point<false, false, PHIMODE, true, 11>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-      asm volatile("" ::: "memory");
-      rhs_point<false, false, PHIMODE, true, 12>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-    } else {
-      rhs_point<false, false, PHIMODE, false, 11>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-      asm volatile("" ::: "memory");
-      rhs_point<false, false, PHIMODE, false, 12>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-    }
+  if (bj == nbj - 1 && j < it.jlo + (nbj - 1) * kTile) return;
+  if (it.skip && i <= it.sihi && j >= it.sjlo && j <= it.sjhi) return;
+  const RoleView V{corner_of(tile, di + kHalo, dj + kHalo), i - kHalo, j - kHalo, kTileW, kTileSize,
+                   rinv + di + kHalo, SHIFT ? shift_slot(SH_dtbeta_r) : 0, nf};
+  const double* const yp = gmem(it.yp);
+  double* const acc = gmem(it.acc);
+  double* const yout = gmem(it.yout);
+  constexpr int R0 = kRole0<SHIFT, SCALAR>, R1 = kRole1<SHIFT, SCALAR>;
+  const bool inside = interior_tile(G, i0, j0);
+  if (__builtin_amdgcn_readfirstlane(tid >> 8) == 0) {
+    if (inside) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
   } else {
-    if (interior_tile(G, i0, j0))
-      rhs_point<false, false, PHIMODE, true, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-    else
-      rhs_point<false, false, PHIMODE, false, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
+    if (inside) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
   }
-  asm volatile("" ::: "memory");
-  rhs_point<SHIFT, SCALAR, PHIMODE, false, 2>(G, it.P, S, V, gmem(it.yp), gmem(it.acc), gmem(it.yout), gaux, i, j);
 }
 
 // Workgroups are dispatched to the 8 XCDs round robin (block b to XCD b % 8),
@@ -222,8 +195,7 @@ __device__ __forceinline__ int xcd_block(int b, int total) {
 }
 
 template <bool SHIFT, bool SCALAR, bool PHIMODE>
-__global__ void __launch_bounds__(kTile * kTile, (kRhsBlocksPerCu<SHIFT, SCALAR>)) k_rhs_table(const RhsItem* __restrict__ items, int n,
-                                                                int xcd_remap) {
+__global__ void __launch_bounds__(kRhsBlock, 4) k_rhs_table(const RhsItem* __restrict__ items, int n, int xcd_remap) {
   extern __shared__ double tile[];
   const int b = xcd_remap ? xcd_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))
                           : static_cast<int>(blockIdx.x);
@@ -232,9 +204,119 @@ __global__ void __launch_bounds__(kTile * kTile, (kRhsBlocksPerCu<SHIFT, SCALAR>
   rhs_tile<SHIFT, SCALAR, PHIMODE>(it, t / it.nbj, t % it.nbj, tile);
 }
 
+// The tile points of a block of 256 threads: each owns q0 = tid and q1 = tid
+// + 256 of the tile's 484.
+struct PhaseSlots {
+  long o0, o1;          // plane offsets of the two points
+  int q0, q1;           // their tile positions
+  bool two;             // q1 lies inside the tile
+};
+
+__device__ __forceinline__ PhaseSlots phase_slots(const KGrid& G, int ib, int jb) {
+  PhaseSlots s;
+  const int tid = static_cast<int>(threadIdx.y) * kTile + static_cast<int>(threadIdx.x);
+  const int lo = 1 - G.g;
+  s.q0 = tid;
+  s.q1 = tid + kTile * kTile;
+  s.two = s.q1 < kTileSize;
+  auto offset = [&](int q) {
+    const int ii = min(max(ib + q / kTileW, lo), G.Nr), jj = min(max(jb + q % kTileW, lo), G.Nz);
+    return IDX(G, ii, jj);
+  };
+  s.o0 = offset(s.q0);
+  s.o1 = s.two ? offset(s.q1) : s.o0;
+  return s;
+}
+
+// the same staging with two points per thread
+template <int NST, class Src>
+__device__ __forceinline__ void stage_planes(double* tile, int first, const PhaseSlots& s, Src src) {
+  double v0[NST], v1[NST];
+#pragma unroll
+  for (int f = 0; f < NST; ++f) {
+    const double* __restrict__ p = src(f);
+    v0[f] = p[s.o0];
+    v1[f] = p[s.o1];
+  }
+#pragma unroll
+  for (int f = 0; f < NST; ++f) {
+    double* dst = tile + (first + f) * kTileSize;
+    dst[s.q0] = v0[f];
+    if (s.two) dst[s.q1] = v1[f];
+  }
+}
+
+// The Gamma-driver in vacuum: one thread per point in two phases.  Phase 1
+// forms the geometric auxiliaries (the Ricci tensor and div KT: the longest
+// expressions, which need only the vacuum fields) and passes them through the
+// per-level buffer gaux; phase 2 forms D_i D_j alpha, every source, the
+// dissipation, the radiative boundaries and the RK update.  Kept apart, the
+// phases need at most the registers of the larger one: 250 VGPRs, two waves
+// per SIMD, and the staged tile (17 fields, 66 KB) allows two blocks per CU.
+// The roles' kernel is faster here too (a Brill step on 5 levels of 256x512
+// at 4.5 ms with it), but it rounds differently, and the constraints of such
+// data, residuals that amplify the last bit of the state by 1/h^2, then move
+// by up to 3e-9 of their size: this configuration keeps its bits.
+// Whether the point lies in an interior tile of the level's whole tile grid.
+// The two forms of phase 1 contract their sums differently, so a point keeps
+// one form whichever range of the level an item computes.
+__device__ __forceinline__ bool interior_point(const KGrid& G, int i, int j) {
+  const int nbi = (G.Nr + kTile - 1) / kTile, nbj = (G.Nz - G.jlo + kTile) / kTile;
+  const int bi = min((i - 1) / kTile, nbi - 1), bj = min((j - G.jlo) / kTile, nbj - 1);
+  return interior_tile(G, tile_start(bi, nbi, 1, G.Nr), tile_start(bj, nbj, G.jlo, G.Nz));
+}
+
+template <bool PHIMODE>
+__device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int bi, int bj, double* tile) {
+  constexpr int nf = nslots(true, false);
+  const KGrid& G = it.G;
+  KStep S = it.S;
+  S.dtb_pre = gmem(S.dtb_pre);            // null stays null
+  const int nbj = it.nbj, nbi = it.nbi;
+  const int j0 = tile_start(bj, nbj, it.jlo, it.jhi);
+  const int i0 = tile_start(bi, nbi, 1, it.ihi);
+  const int ib = i0 - kHalo, jb = j0 - kHalo;
+  if (it.skip && i0 + kTile - 1 <= it.sihi && j0 >= it.sjlo && j0 + kTile - 1 <= it.sjhi) return;
+  // the evolved fields, then (first substep only) the dtbeta planes it differentiates
+  const double* __restrict__ yin = gmem(it.yin);
+  double* const gaux = gmem(it.gaux);
+  {
+    const PhaseSlots ss = phase_slots(G, ib, jb);
+    stage_planes<nf>(tile, 0, ss, [&](int f) { return yin + f * G.plane; });
+    if (S.dtb_pre) stage_planes<2>(tile, nf, ss, [&](int f) { return S.dtb_pre + f * G.plane; });
+    __syncthreads();
+  }
+  const int i = i0 + static_cast<int>(threadIdx.y), j = j0 + static_cast<int>(threadIdx.x);
+  if (bi == nbi - 1 && i < 1 + (nbi - 1) * kTile) return;        // done by the tile before
+  if (bj == nbj - 1 && j < it.jlo + (nbj - 1) * kTile) return;
+  if (it.skip && i <= it.sihi && j >= it.sjlo && j <= it.sjhi) return;
+  const TileView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, nf};
+  // phase 1: the geometric auxiliaries of this point, through gaux (own point
+  // only, so no synchronisation); the memory barrier keeps the compiler from
+  // carrying phase-1 values or loads into phase 2, so the two phases do not
+  // add up in registers
+  if (interior_point(G, i, j))
+    rhs_point<false, PHIMODE, true, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
+  else
+    rhs_point<false, PHIMODE, false, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
+  asm volatile("" ::: "memory");
+  rhs_point<true, PHIMODE, false, 2>(G, it.P, S, V, gmem(it.yp), gmem(it.acc), gmem(it.yout), gaux, i, j);
+}
+
+template <bool PHIMODE>
+__global__ void __launch_bounds__(kTile * kTile, 2) k_rhs_phases(const RhsItem* __restrict__ items, int n,
+                                                                 int xcd_remap) {
+  extern __shared__ double tile[];
+  const int b = xcd_remap ? xcd_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))
+                          : static_cast<int>(blockIdx.x);
+  const RhsItem& it = find_item(items, n, b);
+  const int t = b - it.block0;
+  rhs_phases_tile<PHIMODE>(it, t / it.nbj, t % it.nbj, tile);
+}
+
 // ------------------------------------------------------ constraints
-// The geometric auxiliaries of the current state (phase 1 of the RHS kernel
-// alone, on the vacuum fields), for the constraints.
+// The geometric auxiliaries of the current state (phase 1 of the two-phase
+// kernel alone, on the vacuum fields), for the constraints.
 template <bool PHIMODE>
 __global__ void __launch_bounds__(kTile * kTile, 2) k_aux(RhsItem it) {
   extern __shared__ double tile[];
@@ -244,16 +326,16 @@ __global__ void __launch_bounds__(kTile * kTile, 2) k_aux(RhsItem it) {
   const int i0 = tile_start(bi, it.nbi, 1, G.Nr);
   const int ib = i0 - kHalo, jb = j0 - kHalo;
   const double* __restrict__ yin = it.yin;
-  stage_planes<NBASE>(tile, 0, stage_slots(G, ib, jb), [&](int f) { return yin + f * G.plane; });
+  stage_planes<NBASE>(tile, 0, phase_slots(G, ib, jb), [&](int f) { return yin + f * G.plane; });
   __syncthreads();
   const int i = i0 + static_cast<int>(threadIdx.y), j = j0 + static_cast<int>(threadIdx.x);
   if (bi == it.nbi - 1 && i < 1 + (it.nbi - 1) * kTile) return;     // done by the tile before
   if (bj == it.nbj - 1 && j < G.jlo + (it.nbj - 1) * kTile) return;
   const TileView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, NBASE};
   if (interior_tile(G, i0, j0))
-    rhs_point<false, false, PHIMODE, true, 1>(G, it.P, it.S, V, nullptr, nullptr, nullptr, it.gaux, i, j);
+    rhs_point<false, PHIMODE, true, 1>(G, it.P, it.S, V, nullptr, nullptr, nullptr, it.gaux, i, j);
   else
-    rhs_point<false, false, PHIMODE, false, 1>(G, it.P, it.S, V, nullptr, nullptr, nullptr, it.gaux, i, j);
+    rhs_point<false, PHIMODE, false, 1>(G, it.P, it.S, V, nullptr, nullptr, nullptr, it.gaux, i, j);
 }
 
 struct ConsArgs {
@@ -503,15 +585,64 @@ static int check_launch() {
 
 static int blocks_for(long threads) { return static_cast<int>((threads + kPtBlock - 1) / kPtBlock); }
 
-int rhs_tiles(const KGrid& G, int* nbi, int* nbj) {
-  const int nj = G.Nz - G.jlo + 1;
-  if (G.Nr < kTile || nj < kTile) {
+static void set_tiles(RhsItem* it) {
+  it->nbi = (it->ihi + kTile - 1) / kTile;
+  it->nbj = (it->jhi - it->jlo + 1 + kTile - 1) / kTile;
+}
+
+int rhs_tiles(RhsItem* it, bool* inner) {
+  const KGrid& G = it->G;
+  if (G.Nr < kTile || G.Nz - G.jlo + 1 < kTile) {
     oa_set_error("RHS kernel: a level needs at least 16 points in each direction");
     return OA_ERR_ARG;
   }
-  *nbi = (G.Nr + kTile - 1) / kTile;
-  *nbj = (nj + kTile - 1) / kTile;
+  it->ihi = G.Nr;
+  it->jlo = G.jlo;
+  it->jhi = G.Nz;
+  it->skip = 0;
+  if (*inner) {
+    const int jlo = G.eqsym ? G.jlo : G.jlo + G.g;
+    if (G.Nr - G.g >= kTile && G.Nz - G.g - jlo + 1 >= kTile) {
+      it->ihi = G.Nr - G.g;
+      it->jlo = jlo;
+      it->jhi = G.Nz - G.g;
+    } else {
+      *inner = false;
+    }
+  }
+  set_tiles(it);
   return OA_OK;
+}
+
+RhsItem rhs_frame(const RhsItem& it) {
+  RhsItem f = it;
+  f.skip = 1;
+  f.sihi = it.ihi;
+  f.sjlo = it.jlo;
+  f.sjhi = it.jhi;
+  f.ihi = it.G.Nr;
+  f.jlo = it.G.jlo;
+  f.jhi = it.G.Nz;
+  set_tiles(&f);
+  return f;
+}
+
+void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W) {
+  W->r12 = G.idr / 12.0;
+  W->z12 = G.idz / 12.0;
+  W->rr12 = G.idr * G.idr / 12.0;
+  W->zz12 = G.idz * G.idz / 12.0;
+  W->rz3 = G.idr * G.idz / 3.0;
+  W->rz48 = G.idr * G.idz / 48.0;
+  const double up[3] = {10.5, -3.0, 0.5}, cen[3] = {8.0, -1.0, 0.0};
+  for (int k = 0; k < 3; ++k) {
+    W->ar[k] = (P.shiftadvect ? up[k] : cen[k]) * G.idr / 12.0;
+    W->az[k] = (P.shiftadvect ? up[k] : cen[k]) * G.idz / 12.0;
+  }
+  W->ur = P.shiftadvect ? 0.5 * G.idr / 12.0 : 0.0;
+  W->uz = P.shiftadvect ? 0.5 * G.idz / 12.0 : 0.0;
+  W->ko_g = P.geodiss / G.dt * 0.05;
+  W->ko_s = P.scalardiss / G.dt * 0.05;
 }
 
 int rhs_blocks(const RhsItem& it) { return it.nbi * it.nbj; }
@@ -543,13 +674,15 @@ static int raise_lds_limit(K* kernel, size_t bytes) {
 // planes on a level's first substep (KStep::dtb_pre)
 template <bool SH, bool SC, bool PM>
 static int rhs_lds(bool dtb_pre, size_t* lds) {
-  const size_t per = sizeof(double) * kTileSize;
+  const size_t per = sizeof(double) * kTileSize, col = (SH && !SC) ? 0 : sizeof(double) * kTileW;
   static bool attr_set = false;
   if (!attr_set) {
-    RC_K(raise_lds_limit(&k_rhs_table<SH, SC, PM>, per * static_cast<size_t>(nslots(SH, SC) + 2)));
+    const size_t most = per * static_cast<size_t>(nslots(SH, SC) + 2) + col;
+    if constexpr (SH && !SC) RC_K(raise_lds_limit(&k_rhs_phases<PM>, most));
+    else RC_K(raise_lds_limit(&k_rhs_table<SH, SC, PM>, most));
     attr_set = true;
   }
-  *lds = per * static_cast<size_t>(nslots(SH, SC) + (dtb_pre ? 2 : 0));
+  *lds = per * static_cast<size_t>(nslots(SH, SC) + (dtb_pre ? 2 : 0)) + col;
   return OA_OK;
 }
 
@@ -557,8 +690,13 @@ template <bool SH, bool SC, bool PM>
 static int launch_rhs_table_t(const RhsItem* items, int n, int blocks, bool any_pre, bool xcd, hipStream_t st) {
   size_t lds = 0;
   RC_K((rhs_lds<SH, SC, PM>(any_pre, &lds)));
-  hipLaunchKernelGGL((k_rhs_table<SH, SC, PM>), dim3(blocks), dim3(kTile, kTile, 1), lds, st, items, n, xcd ? 1 : 0);
-  return check_launch();
+  if constexpr (SH && !SC) {
+    hipLaunchKernelGGL((k_rhs_phases<PM>), dim3(blocks), dim3(kTile, kTile, 1), lds, st, items, n, xcd ? 1 : 0);
+    return check_launch();
+  } else {
+    hipLaunchKernelGGL((k_rhs_table<SH, SC, PM>), dim3(blocks), dim3(kRhsBlock), lds, st, items, n, xcd ? 1 : 0);
+    return check_launch();
+  }
 }
 
 // The LDS limits of every RHS variant, raised once before any launch (and so
@@ -720,9 +858,11 @@ int launch_constraints(const KGrid& G, const KPhys& P, const KStep& S, bool phim
                        const double* y, double* gaux, double* out, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   RhsItem it{};
-  RC_K(rhs_tiles(G, &it.nbi, &it.nbj));
   it.G = G;
   it.P = P;
+  bool inner = false;
+  RC_K(rhs_tiles(&it, &inner));
+  rhs_stencil(G, P, &it.W);
   it.S = S;
   it.S.dtb_pre = nullptr;
   it.yin = y;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <string>
+#include <vector>
 
 #include "oaxis.h"
 
@@ -111,12 +112,14 @@ size_t fb_record_bytes();                     // sizeof(FbPoint)
 struct RhsItem {                  // one RK substep of a level
   KGrid G; KPhys P; KStep S; KStencil W;
   const double* yin; const double* yp; double* acc; double* yout; double* gaux;
-  // the computed points: i in [1, ihi], j in [jlo, jhi]; with skip, those of
-  // the frame around i <= sihi, j in [sjlo, sjhi] alone
+  // the computed points: i in [1, ihi], j in [jlo, jhi] in 16 x 16 tiles, nbi
+  // along r and nbj along z, and nstr + nstz per z side strips of the frame
+  // around them.  With skip (two-phase kernel): the frame around i <= sihi, j
+  // in [sjlo, sjhi] alone, in tiles over the whole level
   int ihi, jlo, jhi;
   int skip, sihi, sjlo, sjhi;
-  int nbi, nbj;                   // 16 x 16 tiles along r and z
-  int block0;
+  int nbi, nbj, nstr, nstz;
+  int block0, strip0;             // first tile and first strip of the item
 };
 struct ProjItem {                 // state projection (chi/phi, factordet) of a level
   KGrid G; KPhys P; int time0; double* y;
@@ -154,13 +157,16 @@ int fb_blocks(const FbItem& it, bool shift, bool scalar);
 int rs_blocks(const RsItem& it);
 // The computed points and tiles of a level for the RHS kernel; OA_ERR_ARG if
 // a direction has fewer than 16 points.  inner: without the outer 3 rows,
-// which finebound fills after every substep of a fine level.  Where the rest
-// would have fewer than 16 points in a direction the whole level is taken
-// (*inner set to false).
-int rhs_tiles(RhsItem* it, bool* inner);
-// the frame left out by it, an item with inner tiles: the same substep on
-// the outer rows alone
-RhsItem rhs_frame(const RhsItem& it);
+// which finebound fills after every substep of a fine level; else, where
+// strips are taken (rhs_by_parts), those rows are strips.  Where the rest
+// would have fewer than 16 points in a direction the whole level is taken in
+// tiles (*inner set to false).
+int rhs_tiles(RhsItem* it, bool strips, bool* inner);
+// adds the frame that *items, one item with inner set, leaves out: the same
+// substep on the outer rows
+void rhs_add_frame(std::vector<RhsItem>* items, bool strips);
+bool rhs_by_parts(bool shift, bool scalar);   // the kernel by parts serves these fields
+int rhs_strips(const RhsItem& it);            // strips of an item
 // stencil weights of a level
 void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W);
 
@@ -170,7 +176,8 @@ int prepare_rhs_kernels();
 // launchers (oaxis_kernels.hip): n items in device memory whose block0
 // fields are the prefix sums of their blocks, and the total
 // xcd_remap: renumber blocks so that each XCD takes one contiguous range of tiles
-int launch_rhs_table(const RhsItem* items, int n, int blocks, bool shift, bool scalar, bool phimode,
+// strips: how many of the blocks are frame strips
+int launch_rhs_table(const RhsItem* items, int n, int blocks, int strips, bool shift, bool scalar, bool phimode,
                      bool any_dtb_pre, bool xcd_remap, void* stream);
 int launch_project_table(const ProjItem* items, int n, int blocks, bool shift, bool scalar, void* stream);
 int launch_deldef_table(const DelItem* items, int n, int blocks, void* stream);

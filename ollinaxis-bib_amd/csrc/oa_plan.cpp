@@ -36,8 +36,8 @@ int issue(const LaunchRec& r, const char* dev, bool xcd, hipStream_t st) {
   switch (r.kind) {
     case K_SAVE: return launch_saveold_table(reinterpret_cast<const SaveItem*>(base), r.n, r.blocks, st);
     case K_RHS:
-      return launch_rhs_table(reinterpret_cast<const RhsItem*>(base), r.n, r.blocks, r.shift, r.scalar, r.phimode,
-                              r.any_pre, xcd, st);
+      return launch_rhs_table(reinterpret_cast<const RhsItem*>(base), r.n, r.blocks, r.strips, r.shift, r.scalar,
+                              r.phimode, r.any_pre, xcd, st);
     case K_FB:
       return launch_finebound_table(reinterpret_cast<const FbItem*>(base), r.n, r.blocks, r.shift, r.scalar, st);
     case K_DEL: return launch_deldef_table(reinterpret_cast<const DelItem*>(base), r.n, r.blocks, st);
@@ -67,7 +67,8 @@ bool same_launches(const std::vector<LaunchRec>& a, const std::vector<LaunchRec>
   for (size_t q = 0; q < a.size(); ++q) {
     const LaunchRec &x = a[q], &y = b[q];
     if (x.kind != y.kind || x.shift != y.shift || x.scalar != y.scalar || x.phimode != y.phimode ||
-        x.offset != y.offset || x.n != y.n || x.blocks != y.blocks || x.any_pre != y.any_pre)
+        x.offset != y.offset || x.n != y.n || x.blocks != y.blocks || x.strips != y.strips ||
+        x.any_pre != y.any_pre)
       return false;
   }
   return true;

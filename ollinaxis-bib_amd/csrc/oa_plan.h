@@ -26,6 +26,7 @@ struct LaunchRec {
   size_t offset;    // bytes into the arena
   int n;            // items
   int blocks;       // total blocks
+  int strips;       // RHS: how many of them are frame strips
   bool any_pre;     // an RHS item stages the pre-initialisation dtbeta
   double points;    // RHS: grid points (Nr x Nz) the launch advances one substep
 };
@@ -113,16 +114,19 @@ struct Plan {
       it.block0 = total;
       total += blocks_of(it, shift, scalar);
     }
+    int strips = 0;
     if constexpr (std::is_same<Item, RhsItem>::value)
-      for (const Item& it : items) {
+      for (Item& it : items) {
+        it.strip0 = strips;
+        strips += rhs_strips(it);
         any_pre = any_pre || (it.S.dtb_pre != nullptr);
         points += static_cast<double>(it.G.Nr) * static_cast<double>(it.G.Nz);
       }
     const size_t off = (arena.size() + kAlign - 1) / kAlign * kAlign;
     arena.resize(off + sizeof(Item) * items.size());
     std::memcpy(arena.data() + off, items.data(), sizeof(Item) * items.size());
-    launches.push_back(LaunchRec{kind, shift, scalar, phimode, off, static_cast<int>(items.size()), total,
-                                 any_pre, points});
+    launches.push_back(LaunchRec{kind, shift, scalar, phimode, off, static_cast<int>(items.size()),
+                                 total + strips, strips, any_pre, points});
   }
   template <class Item>
   void add_one(int kind, bool shift, bool scalar, bool phimode, const Item& it) {

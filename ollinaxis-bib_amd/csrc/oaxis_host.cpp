@@ -178,7 +178,7 @@ int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, do
   // its outer ghost-width rows, and nothing reads them (or their accumulator)
   // in between: the substep computes the points inside them
   *inner = level > 0;
-  RC(rhs_tiles(it, inner));
+  RC(rhs_tiles(it, rhs_by_parts(h->shift, h->scalar), inner));
   const int a = L.step_a;
   const int in = (iter == 1) ? a : L.last_out;
   int out;
@@ -338,7 +338,7 @@ int do_substep(oa_handle* h, int level, int iter, int niter, double dtw, double 
   h->plan.begin();
   // on its own a substep leaves every point advanced: the outer rows too
   std::vector<RhsItem> items(1, it);
-  if (inner) items.push_back(rhs_frame(it));
+  if (inner) rhs_add_frame(&items, rhs_by_parts(h->shift, h->scalar));
   h->plan.add(K_RHS, h->shift, h->scalar, phimode, items);
   return h->plan.submit(h->stream);
 }

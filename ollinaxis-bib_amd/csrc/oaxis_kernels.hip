@@ -66,9 +66,9 @@ __device__ __forceinline__ bool interior_tile(const KGrid& G, int i0, int j0) {
 // Points of the tile outside the level, which no stencil reads, take the
 // value of the nearest point inside it, so that every load is in bounds and
 // none needs a branch.
-__device__ __forceinline__ long stage_offset(const KGrid& G, int ib, int jb, int q) {
+__device__ __forceinline__ long stage_offset(const KGrid& G, int ib, int jb, int tw, int q) {
   const int lo = 1 - G.g;
-  const int ii = min(max(ib + q / kTileW, lo), G.Nr), jj = min(max(jb + q % kTileW, lo), G.Nz);
+  const int ii = min(max(ib + q / tw, lo), G.Nr), jj = min(max(jb + q % tw, lo), G.Nz);
   return IDX(G, ii, jj);
 }
 
@@ -110,22 +110,26 @@ __device__ __forceinline__ const double* corner_of(const double* tile, int di, i
   return (const double*)l;
 }
 
-// the item of block b in a table launch: the last one whose block0 <= b
-// (block0 ascends; the loads are uniform across the block)
-template <class Item>
+// the item of block b in a table launch: the last one whose block0 (STRIP:
+// strip0) <= b (they ascend; the loads are uniform across the block)
+template <bool STRIP = false, class Item>
 __device__ __forceinline__ const Item& find_item(const Item* __restrict__ items, int n, int b) {
   int lo = 0, hi = n - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (items[mid].block0 <= b) lo = mid;
+    int first;
+    if constexpr (STRIP) first = items[mid].strip0;
+    else first = items[mid].block0;
+    if (first <= b) lo = mid;
     else hi = mid - 1;
   }
   return items[lo];
 }
 
-// the 1/r column table of a tile, in LDS after its planes
+// the 1/r table of a tile's columns, in LDS after its planes
+constexpr int kInvR = 72;
 __device__ __forceinline__ void stage_inv_r(const KGrid& G, double* rinv, int ib, int q) {
-  if (q < kTileW) rinv[q] = 1.0 / ((static_cast<double>(ib + q) - 0.5) * G.dr);
+  if (q < kInvR) rinv[q] = 1.0 / ((static_cast<double>(ib + q) - 0.5) * G.dr);
 }
 
 // One RK substep of a level.  A block stages its tile once and eight waves
@@ -138,47 +142,88 @@ constexpr int kRole0 = ROLE_K | (SHIFT && SCALAR ? ROLE_SCALAR : SHIFT || SCALAR
 template <bool SHIFT, bool SCALAR>
 constexpr int kRole1 = (ROLE_DELTA | ROLE_LAPSE | ROLE_METRIC | ROLE_SCALAR) & ~kRole0<SHIFT, SCALAR>;
 
+// What a block computes: the 16 x 16 tiles of the item's range, or a strip of
+// the frame around it, the outer 3 rows where some stencils are one-sided:
+//   rho strips  i = Nr-2 .. Nr, 64 points along z; wave w holds row Nr-2+w
+//   z strips    j = Nz-2 .. Nz or j = 1-ghost .. 3-ghost, 62 points along
+//               rho with i <= Nr-3; wave w holds one j
+// so a wave's points share their distance from the edge and take one branch
+// of every closure.  (In square tiles along the edges, each wave ran most
+// branches, three to four times the work of a tile inside.)  Strips stage 6
+// rows or columns: the closures reach 5 points inward.
+constexpr int kStripR = 64, kStripZ = 62;
+constexpr int kStripRW = kStripR + 2 * kHalo, kStripZW = 7;
+static_assert(6 * kStripRW <= kTileSize && (kStripZ + 2 * kHalo) * kStripZW <= kTileSize, "a strip fits the tile's LDS");
+static_assert(kStripZ + 2 * kHalo <= kInvR && kTileW <= kInvR, "1/r table");
+
 template <bool SHIFT, bool SCALAR, bool PHIMODE>
-__device__ __forceinline__ void rhs_tile(const RhsItem& it, int bi, int bj, double* tile) {
+__device__ __forceinline__ void rhs_block(const RhsItem& it, bool strip, int t, double* tile) {
   constexpr int nf = nslots(SHIFT, SCALAR);
   const KGrid& G = it.G;
   KStep S = it.S;
   S.dtb_pre = gmem(S.dtb_pre);            // null stays null
-  const int nbj = it.nbj, nbi = it.nbi;
-  const int j0 = tile_start(bj, nbj, it.jlo, it.jhi);
-  const int i0 = tile_start(bi, nbi, 1, it.ihi);
-  const int ib = i0 - kHalo, jb = j0 - kHalo;
-  if (it.skip && i0 + kTile - 1 <= it.sihi && j0 >= it.sjlo && j0 + kTile - 1 <= it.sjhi) return;
   const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & 63, w = (tid >> 6) & 3;
+  int ib, jb, tw = kTileW, size = kTileSize;   // staged corner, pitch and values
+  int i, j;                                    // this thread's point
+  bool mine = true, inside = false;
+  if (strip) {
+    if (t < it.nstr) {
+      const int js = (t > 0 && t == it.nstr - 1) ? G.Nz - (kStripR - 1) : G.jlo + t * kStripR;
+      ib = G.Nr - 5;
+      jb = js - kHalo;
+      tw = kStripRW;
+      size = 6 * kStripRW;
+      i = G.Nr - 2 + w;
+      j = js + lane;
+      mine = w < 3 && j <= G.Nz && !(t == it.nstr - 1 && j < G.jlo + t * kStripR);
+    } else {
+      const int q = t - it.nstr, side = q / it.nstz, is = 1 + (q % it.nstz) * kStripZ;
+      ib = is - kHalo;
+      jb = side == 0 ? G.Nz - 5 : G.jlo;
+      tw = kStripZW;
+      size = (kStripZ + 2 * kHalo) * kStripZW;
+      i = is + lane;
+      j = (side == 0 ? G.Nz - 2 : G.jlo) + w;
+      mine = w < 3 && lane < kStripZ && i <= G.Nr - 3;
+    }
+  } else {
+    const int bi = t / it.nbj, bj = t % it.nbj;
+    const int i0 = tile_start(bi, it.nbi, 1, it.ihi), j0 = tile_start(bj, it.nbj, it.jlo, it.jhi);
+    ib = i0 - kHalo;
+    jb = j0 - kHalo;
+    i = i0 + 4 * w + lane / kTile;
+    j = j0 + lane % kTile;
+    inside = interior_tile(G, i0, j0);
+    // points of the last tile that the tile before it covers
+    mine = !(bi == it.nbi - 1 && i < 1 + bi * kTile) && !(bj == it.nbj - 1 && j < it.jlo + bj * kTile);
+  }
   // the evolved fields, then (first substep only) the dtbeta planes it
   // differentiates, then the 1/r table
   const double* __restrict__ yin = gmem(it.yin);
   double* const rinv = tile + (nf + (SHIFT && S.dtb_pre ? 2 : 0)) * kTileSize;
-  if (tid < kTileSize) {
-    const long off = stage_offset(G, ib, jb, tid);
+  if (tid < size) {
+    const long off = stage_offset(G, ib, jb, tw, tid);
     stage_planes<nf>(tile, 0, tid, off, [&](int f) { return yin + f * G.plane; });
     if (SHIFT && S.dtb_pre) stage_planes<2>(tile, nf, tid, off, [&](int f) { return S.dtb_pre + f * G.plane; });
   }
   stage_inv_r(G, rinv, ib, tid);
   __syncthreads();
-  const int p = tid & 255;
-  const int di = p / kTile, dj = p % kTile;
-  const int i = i0 + di, j = j0 + dj;
-  if (bi == nbi - 1 && i < 1 + (nbi - 1) * kTile) return;        // done by the tile before
-  if (bj == nbj - 1 && j < it.jlo + (nbj - 1) * kTile) return;
-  if (it.skip && i <= it.sihi && j >= it.sjlo && j <= it.sjhi) return;
-  const RoleView V{corner_of(tile, di + kHalo, dj + kHalo), i - kHalo, j - kHalo, kTileW, kTileSize,
-                   rinv + di + kHalo, SHIFT ? shift_slot(SH_dtbeta_r) : 0, nf};
+  if (!mine) return;
   const double* const yp = gmem(it.yp);
   double* const acc = gmem(it.acc);
   double* const yout = gmem(it.yout);
   constexpr int R0 = kRole0<SHIFT, SCALAR>, R1 = kRole1<SHIFT, SCALAR>;
-  const bool inside = interior_tile(G, i0, j0);
-  if (__builtin_amdgcn_readfirstlane(tid >> 8) == 0) {
-    if (inside) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
-    else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+  constexpr int ndtb = SHIFT ? shift_slot(SH_dtbeta_r) : 0;
+  const double* const ri = rinv + (i - ib);
+  const bool second = __builtin_amdgcn_readfirstlane(tid >> 8) != 0;
+  if (inside) {
+    const RoleView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, ri, ndtb, nf};
+    if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    else rhs_roles<SHIFT, SCALAR, PHIMODE, true, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
   } else {
-    if (inside) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    const RoleView V{tile + (i - ib) * tw + (j - jb), i, j, tw, kTileSize, ri, ndtb, nf};
+    if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, false, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
     else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
   }
 }
@@ -194,14 +239,21 @@ __device__ __forceinline__ int xcd_block(int b, int total) {
   return x * q + (x < r ? x : r) + l;
 }
 
+// The first `strips` blocks are the items' frame strips, which take longer than
+// a tile inside: they start first and are spread over the XCDs.
 template <bool SHIFT, bool SCALAR, bool PHIMODE>
-__global__ void __launch_bounds__(kRhsBlock, 4) k_rhs_table(const RhsItem* __restrict__ items, int n, int xcd_remap) {
+__global__ void __launch_bounds__(kRhsBlock, 4) k_rhs_table(const RhsItem* __restrict__ items, int n, int strips,
+                                                            int xcd_remap) {
   extern __shared__ double tile[];
-  const int b = xcd_remap ? xcd_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))
-                          : static_cast<int>(blockIdx.x);
-  const RhsItem& it = find_item(items, n, b);
-  const int t = b - it.block0;
-  rhs_tile<SHIFT, SCALAR, PHIMODE>(it, t / it.nbj, t % it.nbj, tile);
+  const int b = static_cast<int>(blockIdx.x);
+  const bool strip = b < strips;
+  int t = b;
+  if (!strip) {
+    t = b - strips;
+    if (xcd_remap) t = xcd_block(t, static_cast<int>(gridDim.x) - strips);
+  }
+  const RhsItem& it = strip ? find_item<true>(items, n, t) : find_item<false>(items, n, t);
+  rhs_block<SHIFT, SCALAR, PHIMODE>(it, strip, t - (strip ? it.strip0 : it.block0), tile);
 }
 
 // The tile points of a block of 256 threads: each owns q0 = tid and q1 = tid
@@ -590,7 +642,17 @@ static void set_tiles(RhsItem* it) {
   it->nbj = (it->jhi - it->jlo + 1 + kTile - 1) / kTile;
 }
 
-int rhs_tiles(RhsItem* it, bool* inner) {
+static void set_strips(RhsItem* it) {
+  const KGrid& G = it->G;
+  it->nstr = (G.Nz - G.jlo + 1 + kStripR - 1) / kStripR;
+  it->nstz = (G.Nr - G.g + kStripZ - 1) / kStripZ;
+}
+
+bool rhs_by_parts(bool shift, bool scalar) { return !shift || scalar; }
+
+int rhs_strips(const RhsItem& it) { return it.nstr + it.nstz * (it.G.eqsym ? 1 : 2); }
+
+int rhs_tiles(RhsItem* it, bool strips, bool* inner) {
   const KGrid& G = it->G;
   if (G.Nr < kTile || G.Nz - G.jlo + 1 < kTile) {
     oa_set_error("RHS kernel: a level needs at least 16 points in each direction");
@@ -600,12 +662,14 @@ int rhs_tiles(RhsItem* it, bool* inner) {
   it->jlo = G.jlo;
   it->jhi = G.Nz;
   it->skip = 0;
-  if (*inner) {
+  it->nstr = it->nstz = 0;
+  if (*inner || strips) {
     const int jlo = G.eqsym ? G.jlo : G.jlo + G.g;
     if (G.Nr - G.g >= kTile && G.Nz - G.g - jlo + 1 >= kTile) {
       it->ihi = G.Nr - G.g;
       it->jlo = jlo;
       it->jhi = G.Nz - G.g;
+      if (!*inner) set_strips(it);
     } else {
       *inner = false;
     }
@@ -614,7 +678,12 @@ int rhs_tiles(RhsItem* it, bool* inner) {
   return OA_OK;
 }
 
-RhsItem rhs_frame(const RhsItem& it) {
+void rhs_add_frame(std::vector<RhsItem>* items, bool strips) {
+  RhsItem& it = items->front();
+  if (strips) {
+    set_strips(&it);
+    return;
+  }
   RhsItem f = it;
   f.skip = 1;
   f.sihi = it.ihi;
@@ -624,7 +693,7 @@ RhsItem rhs_frame(const RhsItem& it) {
   f.jlo = it.G.jlo;
   f.jhi = it.G.Nz;
   set_tiles(&f);
-  return f;
+  items->push_back(f);
 }
 
 void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W) {
@@ -674,7 +743,7 @@ static int raise_lds_limit(K* kernel, size_t bytes) {
 // planes on a level's first substep (KStep::dtb_pre)
 template <bool SH, bool SC, bool PM>
 static int rhs_lds(bool dtb_pre, size_t* lds) {
-  const size_t per = sizeof(double) * kTileSize, col = (SH && !SC) ? 0 : sizeof(double) * kTileW;
+  const size_t per = sizeof(double) * kTileSize, col = (SH && !SC) ? 0 : sizeof(double) * kInvR;
   static bool attr_set = false;
   if (!attr_set) {
     const size_t most = per * static_cast<size_t>(nslots(SH, SC) + 2) + col;
@@ -687,14 +756,16 @@ static int rhs_lds(bool dtb_pre, size_t* lds) {
 }
 
 template <bool SH, bool SC, bool PM>
-static int launch_rhs_table_t(const RhsItem* items, int n, int blocks, bool any_pre, bool xcd, hipStream_t st) {
+static int launch_rhs_table_t(const RhsItem* items, int n, int blocks, int strips, bool any_pre, bool xcd,
+                              hipStream_t st) {
   size_t lds = 0;
   RC_K((rhs_lds<SH, SC, PM>(any_pre, &lds)));
   if constexpr (SH && !SC) {
+    (void)strips;
     hipLaunchKernelGGL((k_rhs_phases<PM>), dim3(blocks), dim3(kTile, kTile, 1), lds, st, items, n, xcd ? 1 : 0);
     return check_launch();
   } else {
-    hipLaunchKernelGGL((k_rhs_table<SH, SC, PM>), dim3(blocks), dim3(kRhsBlock), lds, st, items, n, xcd ? 1 : 0);
+    hipLaunchKernelGGL((k_rhs_table<SH, SC, PM>), dim3(blocks), dim3(kRhsBlock), lds, st, items, n, strips, xcd ? 1 : 0);
     return check_launch();
   }
 }
@@ -729,10 +800,10 @@ int prepare_rhs_kernels() {
     default: return FN<true, true, true>(__VA_ARGS__);          \
   }
 
-int launch_rhs_table(const RhsItem* items, int n, int blocks, bool shift, bool scalar, bool phimode,
+int launch_rhs_table(const RhsItem* items, int n, int blocks, int strips, bool shift, bool scalar, bool phimode,
                      bool any_dtb_pre, bool xcd_remap, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
-  RHS_DISPATCH(launch_rhs_table_t, items, n, blocks, any_dtb_pre, xcd_remap, st)
+  RHS_DISPATCH(launch_rhs_table_t, items, n, blocks, strips, any_dtb_pre, xcd_remap, st)
 }
 
 #define SC_DISPATCH(K, GRID, ...)                                                                  \
@@ -861,7 +932,7 @@ int launch_constraints(const KGrid& G, const KPhys& P, const KStep& S, bool phim
   it.G = G;
   it.P = P;
   bool inner = false;
-  RC_K(rhs_tiles(&it, &inner));
+  RC_K(rhs_tiles(&it, false, &inner));
   rhs_stencil(G, P, &it.W);
   it.S = S;
   it.S.dtb_pre = nullptr;

@@ -109,6 +109,15 @@ size_t fb_record_bytes();                     // sizeof(FbPoint)
 // launch needs.  Item k owns the blocks [block0, block0 + blocks) of the
 // grid.  A spacetime alone launches tables of one item; a batch of
 // spacetimes launches one table over all its members.
+// The boundary work of a level that rides on a substep's launch: finebound of
+// the substep's output (n > 0) and saveold of the step's start (rR set).
+struct EdgeWork {
+  KGrid Gc; KTime T; int time0;
+  const FbPoint* table; long n;   // the zone's point records
+  const double* yc;
+  const double* rR1; const double* zL1; const double* zR1;   // strips of time level t-1
+  double* rR; double* zL; double* zR;                        // strips saveold fills
+};
 struct RhsItem {                  // one RK substep of a level
   KGrid G; KPhys P; KStep S; KStencil W;
   const double* yin; const double* yp; double* acc; double* yout; double* gaux;
@@ -119,6 +128,10 @@ struct RhsItem {                  // one RK substep of a level
   int ihi, jlo, jhi;
   int skip, sihi, sjlo, sjhi;
   int nbi, nbj, nstr, nstz;
+  // points of the zone finebound fills, of depth `depth`, are left to it
+  int depth;                      // -1: none
+  EdgeWork E;
+  int xtra;                       // blocks for the edge work alone, after the tiles
   int block0, strip0;             // first tile and first strip of the item
 };
 struct ProjItem {                 // state projection (chi/phi, factordet) of a level
@@ -167,6 +180,8 @@ int rhs_tiles(RhsItem* it, bool strips, bool* inner);
 void rhs_add_frame(std::vector<RhsItem>* items, bool strips);
 bool rhs_by_parts(bool shift, bool scalar);   // the kernel by parts serves these fields
 int rhs_strips(const RhsItem& it);            // strips of an item
+// gives the items of a launch blocks of their own for the edge work (xtra)
+void rhs_plan_edges(std::vector<RhsItem>* items, bool shift, bool scalar);
 // stencil weights of a level
 void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W);
 

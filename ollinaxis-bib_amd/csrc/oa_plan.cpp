@@ -47,6 +47,26 @@ int issue(const LaunchRec& r, const char* dev, bool xcd, hipStream_t st) {
   }
 }
 
+void ride_saveold(const SaveItem& s, RhsItem* it) {
+  it->E.rR = s.rR;
+  it->E.zL = s.zL;
+  it->E.zR = s.zR;
+}
+
+void ride_finebound(const FbItem& f, RhsItem* it) {
+  EdgeWork& E = it->E;
+  it->depth = f.T.depth;
+  E.Gc = f.Gc;
+  E.T = f.T;
+  E.time0 = f.time0;
+  E.table = f.table;
+  E.n = f.n;
+  E.yc = f.yc;
+  E.rR1 = f.rR1;
+  E.zL1 = f.zL1;
+  E.zR1 = f.zR1;
+}
+
 int group_code(bool shift, bool scalar) { return (shift ? 2 : 0) + (scalar ? 1 : 0); }
 
 }  // namespace
@@ -291,7 +311,6 @@ int plan_level(Plan& plan, const std::vector<oa_handle*>& all, int level) {
 
   std::vector<SaveItem> sv(nm);
   for (size_t k = 0; k < nm; ++k) RC(prepare_saveold(M[k], level, &sv[k]));
-  plan.add(K_SAVE, false, false, false, sv);
 
   std::vector<char> time0(nm);
   int nmax = 0;
@@ -299,32 +318,31 @@ int plan_level(Plan& plan, const std::vector<oa_handle*>& all, int level) {
     time0[k] = (M[k]->L[level].t == 0.0);
     nmax = std::max(nmax, niter_of(M[k]));
   }
-  std::vector<double> dtws(nm);
   for (int iter = 1; iter <= nmax; ++iter) {
     std::vector<RhsItem> rhs[8];
+    std::vector<FbItem> fb[4];
     for (size_t k = 0; k < nm; ++k) {
       oa_handle* h = M[k];
       const int ni = niter_of(h);
       if (iter > ni) continue;
       double dtw, w;
       substep_weights(h, level, iter, &dtw, &w);
-      dtws[k] = dtw;
       RhsItem it;
       bool pm = false, inner = false;
       RC(prepare_substep(h, level, iter, ni, dtw, w, &it, &pm, &inner));
+      // saveold rides on the first substep, whose input is the step's start
+      if (iter == 1) ride_saveold(sv[k], &it);
+      // finebound rides on the substep whose output it fills, unless the
+      // substep computes the whole of a level too small for inner tiles
+      FbItem f;
+      if (prepare_finebound(h, level, dtw, &f)) {
+        if (inner) ride_finebound(f, &it);
+        else fb[group_code(h->shift, h->scalar)].push_back(f);
+      }
       rhs[group_code(h->shift, h->scalar) * 2 + (pm ? 1 : 0)].push_back(it);
     }
     for (int c = 0; c < 8; ++c) plan.add(K_RHS, (c & 4) != 0, (c & 2) != 0, (c & 1) != 0, rhs[c]);
-    if (level > 0) {
-      std::vector<FbItem> fb[4];
-      for (size_t k = 0; k < nm; ++k) {
-        oa_handle* h = M[k];
-        if (iter > niter_of(h)) continue;
-        FbItem it;
-        if (prepare_finebound(h, level, dtws[k], &it)) fb[group_code(h->shift, h->scalar)].push_back(it);
-      }
-      for (int c = 0; c < 4; ++c) plan.add(K_FB, (c & 2) != 0, (c & 1) != 0, false, fb[c]);
-    }
+    for (int c = 0; c < 4; ++c) plan.add(K_FB, (c & 2) != 0, (c & 1) != 0, false, fb[c]);
     std::vector<DelItem> del;
     for (size_t k = 0; k < nm; ++k) {
       oa_handle* h = M[k];

@@ -110,6 +110,7 @@ struct Plan {
     int total = 0;
     bool any_pre = false;
     double points = 0.0;
+    if constexpr (std::is_same<Item, RhsItem>::value) rhs_plan_edges(&items, shift, scalar);
     for (Item& it : items) {
       it.block0 = total;
       total += blocks_of(it, shift, scalar);

@@ -199,6 +199,22 @@ OA_HD double s_ko(const F& f, const KGrid& G, int i, int j, double dscale) {
   return s + t;
 }
 
+// Between two parts of a long expression: no load moves across it, and the
+// partial results given to it are finished before it.  So the stencil values
+// of one part are in registers at a time; left alone, the compiler reads the
+// stencils of every field first and does the arithmetic last, which spills
+// hundreds of registers.
+OA_HD void finish(double& v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+v"(v));
+#endif
+}
+template <class... T>
+OA_HD void part(T&... v) {
+  (finish(v), ...);
+  asm volatile("" ::: "memory");
+}
+
 struct Plane {
   const double* __restrict__ p;
   KGrid G;
@@ -1130,7 +1146,7 @@ OA_HD void fb_geometry(const KGrid& Gf, const KGrid& Gc, int D, int interporder,
     if (row <= D) { n = row; j = Gf.Nz - n; which = 1; }
     else { n = row - (D + 1); j = 1 - g + n; which = 2; }
   }
-  if (i < 1) return;   // axis images are refreshed by parity
+  if (i < 1 || (Gf.eqsym && j < 1)) return;   // images are refreshed by parity
   // coordinates of the fine point as finebound.f90 forms them
   const double rminf = coord_r(Gf, 1 - g), rmaxf = coord_r(Gf, Gf.Nr);
   const double zminf = coord_z(Gf, 1 - g), zmaxf = coord_z(Gf, Gf.Nz);
@@ -1146,73 +1162,76 @@ OA_HD void fb_geometry(const KGrid& Gf, const KGrid& Gc, int D, int interporder,
   fp.strip_ok = ((which == 0 ? m : n) < g) ? 1 : 0;
 }
 
-template <bool SHIFT, bool SCALAR>
+// Groups of fields a thread takes at a point: the metric, which factordet
+// couples; chi (with phi while it is kept); then every other field alone.
+constexpr int finebound_groups(bool shift, bool scalar) { return 3 + nslots(shift, scalar) - (S_C + 1); }
+
+// b0(s): field s at the point at time level t0 (var_p); r1, zL1, zR1: the
+// strips of time level t-1.  Fields are interpolated two at a time, so that
+// their 32 loads are in flight together and no more registers are held.
+template <bool SHIFT, bool SCALAR, class B0>
 OA_HD void finebound_point(const KGrid& Gf, const KGrid& Gc, const KPhys& P, const KTime& T, int time0,
-                           const double* __restrict__ yc, double* __restrict__ yf,
-                           const double* __restrict__ rR0, const double* __restrict__ rR1,
-                           const double* __restrict__ zL0, const double* __restrict__ zL1,
-                           const double* __restrict__ zR0, const double* __restrict__ zR1, const FbPoint& fp_in,
-                           int grp) {
+                           const double* __restrict__ yc, double* __restrict__ yf, const double* __restrict__ r1,
+                           const double* __restrict__ zL1, const double* __restrict__ zR1, const FbPoint& fp_in,
+                           int grp, const B0& b0) {
   const FbPoint fp = fp_in;   // the whole record in one go
   if (fp.which < 0) return;
   const int g = Gf.g, i = fp.i, j = fp.j;
   const Cell& c = fp.c;
   const long pf = Gf.plane, pc = Gc.plane;
-  // the strip this point belongs to, for the time levels
-  const double* s0 = (fp.which == 0) ? rR0 : (fp.which == 1) ? zR0 : zL0;
-  const double* s1 = (fp.which == 0) ? rR1 : (fp.which == 1) ? zR1 : zL1;
+  // the strip this point belongs to, for the time level t-1
+  const double* s1 = (fp.which == 0) ? r1 : (fp.which == 1) ? zR1 : zL1;
   const long sper = static_cast<long>(g) * ((fp.which == 0) ? (Gf.Nz + g) : (Gf.Nr + g));
   const long sidx = fp.sidx;
   const bool strip_ok = fp.strip_ok != 0;
 
   // time interpolation of one injected value (bound_interp.inc)
-  auto value = [&](int s) -> double {
-    const double aux2 = apply(c, yc + s * pc, Gc);
-    const double b0 = strip_ok ? s0[s * sper + sidx] : 0.0;   // state at t0 (var_p)
-    if (T.border == 1) return T.c_aux * aux2 + (T.same ? 0.0 : T.c_p * b0);
-    const double b1 = strip_ok ? s1[s * sper + sidx] : 0.0;
-    return T.c0 * aux2 + (T.same ? 0.0 : T.c1 * b0 + T.c2 * b1);
+  auto in_time = [&](double aux2, double q0, double q1) -> double {
+    if (T.border == 1) return T.c_aux * aux2 + (T.same ? 0.0 : T.c_p * q0);
+    return T.c0 * aux2 + (T.same ? 0.0 : T.c1 * q0 + T.c2 * q1);
   };
+  auto old0 = [&](int s) { return strip_ok ? b0(s) : 0.0; };
+  auto old1 = [&](int s) { return (strip_ok && T.border != 1) ? s1[s * sper + sidx] : 0.0; };
+  auto value = [&](int s) -> double { return in_time(apply(c, yc + s * pc, Gc), old0(s), old1(s)); };
   if (grp == 0) {
-    // the fields coupled by the projection (chi/phi, factordet) go together;
-    // the six interpolations share one branch on the cell kind and issue
-    // their loads together (value() for each field in turn would wait for
-    // each field's loads before starting the next)
-    constexpr int kN = 6;
-    const int slot[kN] = {S_chi, S_phi, S_A, S_B, S_H, S_C};
-    double v[kN];
-    apply_many<kN>(c, yc, pc, slot, v, Gc);
-    double b0[kN], b1[kN];
-#pragma unroll
-    for (int q = 0; q < kN; ++q) {
-      b0[q] = strip_ok ? s0[slot[q] * sper + sidx] : 0.0;
-      b1[q] = (strip_ok && T.border != 1) ? s1[slot[q] * sper + sidx] : 0.0;
+    Proj q;
+    double v[2];
+    {
+      const int slot[2] = {S_A, S_B};
+      const double p0[2] = {old0(S_A), old0(S_B)}, p1[2] = {old1(S_A), old1(S_B)};
+      apply_many<2>(c, yc, pc, slot, v, Gc);
+      q.A = in_time(v[0], p0[0], p1[0]);
+      q.B = in_time(v[1], p0[1], p1[1]);
     }
-#pragma unroll
-    for (int q = 0; q < kN; ++q) {
-      if (T.border == 1) v[q] = T.c_aux * v[q] + (T.same ? 0.0 : T.c_p * b0[q]);
-      else v[q] = T.c0 * v[q] + (T.same ? 0.0 : T.c1 * b0[q] + T.c2 * b1[q]);
+    part(q.A, q.B);
+    {
+      const int slot[2] = {S_H, S_C};
+      const double p0[2] = {old0(S_H), old0(S_C)}, p1[2] = {old1(S_H), old1(S_C)};
+      apply_many<2>(c, yc, pc, slot, v, Gc);
+      q.H = in_time(v[0], p0[0], p1[0]);
+      q.C = in_time(v[1], p0[1], p1[1]);
     }
-    const double r = coord_r(Gf, i);
-    Proj qp{v[0], v[1], v[2], v[3], v[4], v[5]};
-    project(qp, r, time0 != 0, P.chimethod, SCALAR);
-    put(yf + S_chi * pf, Gf, i, j, qp.chi, 1.0, 1.0);
-    if (time0 || !P.chimethod) put(yf + S_phi * pf, Gf, i, j, qp.phi, 1.0, 1.0);   // phi is not kept after the first step
-    put(yf + S_A * pf, Gf, i, j, qp.A, 1.0, 1.0);
-    put(yf + S_B * pf, Gf, i, j, qp.B, 1.0, 1.0);
-    put(yf + S_H * pf, Gf, i, j, qp.H, 1.0, 1.0);
-    put(yf + S_C * pf, Gf, i, j, qp.C, 1.0, -1.0);
+    if (!time0) factordet(q, coord_r(Gf, i));
+    put(yf + S_A * pf, Gf, i, j, q.A, 1.0, 1.0);
+    put(yf + S_B * pf, Gf, i, j, q.B, 1.0, 1.0);
+    put(yf + S_H * pf, Gf, i, j, q.H, 1.0, 1.0);
+    put(yf + S_C * pf, Gf, i, j, q.C, 1.0, -1.0);
+  } else if (grp == 1) {
+    Proj q;
+    const bool by_phi = time0 || !P.chimethod;   // phi is not kept after the first step
+    if (by_phi) q.phi = value(S_phi);
+    else q.chi = value(S_chi);
+    project_factor(q, time0 != 0, P.chimethod, SCALAR);
+    put(yf + S_chi * pf, Gf, i, j, q.chi, 1.0, 1.0);
+    if (by_phi) put(yf + S_phi * pf, Gf, i, j, q.phi, 1.0, 1.0);
   } else {
-    // every other field on its own: alpha, then the slots after S_C
-    const int s = (grp == 1) ? S_alpha : S_C + grp - 1;
+    // alpha, then the slots after S_C
+    const int s = (grp == 2) ? S_alpha : S_C + grp - 2;
     double symr, symz;
     slot_parity(SHIFT, SCALAR, s, symr, symz);
     put(yf + s * pf, Gf, i, j, value(s), symr, symz);
   }
 }
-
-// groups of finebound_point: the projected set, then one per remaining slot
-constexpr int finebound_groups(bool shift, bool scalar) { return 2 + nslots(shift, scalar) - (S_C + 1); }
 
 // restrict(box 0, level, .true.): coarse points well inside the fine level
 // take the bicubic interpolant of the fine level (restrict.f90:88-162);

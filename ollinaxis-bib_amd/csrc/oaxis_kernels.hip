@@ -49,6 +49,7 @@ constexpr int kTile = 16, kHalo = 3;
 constexpr int kTileW = kTile + 2 * kHalo;                 // staged extent per direction
 constexpr int kTileSize = kTileW * kTileW;                // values per field
 constexpr int kRhsBlock = 512;                            // two waves per 64 points
+constexpr int kResidentBlocks = 512;                      // RHS blocks resident at once (256 CUs x 2)
 
 // first point of tile b of nb along [lo, hi] (extent >= kTile)
 __host__ __device__ inline int tile_start(int b, int nb, int lo, int hi) {
@@ -132,6 +133,57 @@ __device__ __forceinline__ void stage_inv_r(const KGrid& G, double* rinv, int ib
   if (q < kInvR) rinv[q] = 1.0 / ((static_cast<double>(ib + q) - 0.5) * G.dr);
 }
 
+// The boundary work that rides on a substep's launch, in units of one wave:
+// 64 records of one field group of finebound, or 64 points of one field's
+// strips of saveold.  Finebound reads the coarse level, the step's start at
+// its own points and the strips of time level t-1, and writes only the zone,
+// which the substep leaves alone; saveold reads the step's start.  So both run
+// beside the tiles, and a level step is one launch per substep instead of two
+// and a saveold (each a few us that leave most of the GPU idle).
+__device__ __forceinline__ int edge_fb_units(long n, int groups) { return groups * static_cast<int>((n + 63) / 64); }
+
+template <bool SHIFT, bool SCALAR>
+__device__ __forceinline__ void edge_work(const RhsItem& it, int v, int nv) {
+  constexpr int groups = finebound_groups(SHIFT, SCALAR), nf = nslots(SHIFT, SCALAR);
+  const KGrid& G = it.G;
+  const int lane = static_cast<int>(threadIdx.x & 63u);
+  const long n = it.E.n;
+  const int ufb = edge_fb_units(n, groups), chunks = static_cast<int>((n + 63) / 64);
+  const int nrt = G.Nr + G.g, nzt = G.Nz + G.g, per = G.g * max(nrt, nzt), schunks = (per + 63) / 64;
+  const int usave = it.E.rR ? nf * schunks : 0;
+  for (int u = v; u < ufb + usave; u += nv) {
+    if (u < ufb) {
+      const int grp = u / chunks;
+      const long q = static_cast<long>(u % chunks) * 64 + lane;
+      if (q >= n) continue;
+      const double* const yp = gmem(it.yp);
+      const FbPoint* const rec = gmem(it.E.table) + q;
+      const long k = IDX(G, rec->i, rec->j);
+      finebound_point<SHIFT, SCALAR>(G, it.E.Gc, it.P, it.E.T, it.E.time0, gmem(it.E.yc), gmem(it.yout),
+                                     gmem(it.E.rR1), gmem(it.E.zL1), gmem(it.E.zR1), *rec, grp,
+                                     [&](int s) { return yp[s * G.plane + k]; });
+    } else {
+      const int s = u - ufb, f = s / schunks, q = (s % schunks) * 64 + lane;
+      if (q < per) saveold_point(G, gmem(it.yp), gmem(it.E.rR), gmem(it.E.zL), gmem(it.E.zR), f, q);
+    }
+  }
+}
+
+// this wave's share of the edge work of an item with nt tiles: block t of its
+// nt + xtra, wave w of W; its own blocks come first, then wave after wave of
+// the tiles' blocks
+template <bool SHIFT, bool SCALAR>
+__device__ __forceinline__ void edge_share(const RhsItem& it, int nt, int t, int w, int W) {
+  if (it.E.n == 0 && !it.E.rR) return;
+  const int v = t >= nt ? (t - nt) * W + w : it.xtra * W + w * nt + t;
+  edge_work<SHIFT, SCALAR>(it, __builtin_amdgcn_readfirstlane(v), (nt + it.xtra) * W);
+}
+
+// the point is left to finebound (depth < 0: none is)
+__device__ __forceinline__ bool finebound_zone(const KGrid& G, int depth, int i, int j) {
+  return depth >= 0 && (i >= G.Nr - depth || j >= G.Nz - depth || (!G.eqsym && j <= 1 - G.g + depth));
+}
+
 // One RK substep of a level.  A block stages its tile once and eight waves
 // work on it: waves 0-3 form one half of the sources of the tile's points,
 // waves 4-7 the other half (rhs_roles), so the LDS of a tile serves twice the
@@ -187,6 +239,9 @@ __device__ __forceinline__ void rhs_block(const RhsItem& it, bool strip, int t, 
       j = (side == 0 ? G.Nz - 2 : G.jlo) + w;
       mine = w < 3 && lane < kStripZ && i <= G.Nr - 3;
     }
+  } else if (t >= it.nbi * it.nbj) {
+    edge_share<SHIFT, SCALAR>(it, it.nbi * it.nbj, t, tid >> 6, kRhsBlock / 64);
+    return;
   } else {
     const int bi = t / it.nbj, bj = t % it.nbj;
     const int i0 = tile_start(bi, it.nbi, 1, it.ihi), j0 = tile_start(bj, it.nbj, it.jlo, it.jhi);
@@ -196,7 +251,8 @@ __device__ __forceinline__ void rhs_block(const RhsItem& it, bool strip, int t, 
     j = j0 + lane % kTile;
     inside = interior_tile(G, i0, j0);
     // points of the last tile that the tile before it covers
-    mine = !(bi == it.nbi - 1 && i < 1 + bi * kTile) && !(bj == it.nbj - 1 && j < it.jlo + bj * kTile);
+    mine = !(bi == it.nbi - 1 && i < 1 + bi * kTile) && !(bj == it.nbj - 1 && j < it.jlo + bj * kTile) &&
+           !finebound_zone(G, it.depth, i, j);
   }
   // the evolved fields, then (first substep only) the dtbeta planes it
   // differentiates, then the 1/r table
@@ -209,23 +265,25 @@ __device__ __forceinline__ void rhs_block(const RhsItem& it, bool strip, int t, 
   }
   stage_inv_r(G, rinv, ib, tid);
   __syncthreads();
-  if (!mine) return;
-  const double* const yp = gmem(it.yp);
-  double* const acc = gmem(it.acc);
-  double* const yout = gmem(it.yout);
-  constexpr int R0 = kRole0<SHIFT, SCALAR>, R1 = kRole1<SHIFT, SCALAR>;
-  constexpr int ndtb = SHIFT ? shift_slot(SH_dtbeta_r) : 0;
-  const double* const ri = rinv + (i - ib);
   const bool second = __builtin_amdgcn_readfirstlane(tid >> 8) != 0;
-  if (inside) {
-    const RoleView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, ri, ndtb, nf};
-    if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
-    else rhs_roles<SHIFT, SCALAR, PHIMODE, true, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
-  } else {
-    const RoleView V{tile + (i - ib) * tw + (j - jb), i, j, tw, kTileSize, ri, ndtb, nf};
-    if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, false, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
-    else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+  if (mine) {
+    const double* const yp = gmem(it.yp);
+    double* const acc = gmem(it.acc);
+    double* const yout = gmem(it.yout);
+    constexpr int R0 = kRole0<SHIFT, SCALAR>, R1 = kRole1<SHIFT, SCALAR>;
+    constexpr int ndtb = SHIFT ? shift_slot(SH_dtbeta_r) : 0;
+    const double* const ri = rinv + (i - ib);
+    if (inside) {
+      const RoleView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, ri, ndtb, nf};
+      if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, true, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+      else rhs_roles<SHIFT, SCALAR, PHIMODE, true, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    } else {
+      const RoleView V{tile + (i - ib) * tw + (j - jb), i, j, tw, kTileSize, ri, ndtb, nf};
+      if (!second) rhs_roles<SHIFT, SCALAR, PHIMODE, false, R0>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+      else rhs_roles<SHIFT, SCALAR, PHIMODE, false, R1>(G, it.P, S, it.W, V, yp, acc, yout, i, j);
+    }
   }
+  if (!strip) edge_share<SHIFT, SCALAR>(it, it.nbi * it.nbj, t, 7 - (tid >> 6), kRhsBlock / 64);
 }
 
 // Workgroups are dispatched to the 8 XCDs round robin (block b to XCD b % 8),
@@ -266,7 +324,7 @@ struct PhaseSlots {
 
 __device__ __forceinline__ PhaseSlots phase_slots(const KGrid& G, int ib, int jb) {
   PhaseSlots s;
-  const int tid = static_cast<int>(threadIdx.y) * kTile + static_cast<int>(threadIdx.x);
+  const int tid = static_cast<int>(threadIdx.y * blockDim.x + threadIdx.x);
   const int lo = 1 - G.g;
   s.q0 = tid;
   s.q1 = tid + kTile * kTile;
@@ -319,9 +377,16 @@ __device__ __forceinline__ bool interior_point(const KGrid& G, int i, int j) {
 }
 
 template <bool PHIMODE>
-__device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int bi, int bj, double* tile) {
+__device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int t, double* tile) {
   constexpr int nf = nslots(true, false);
   const KGrid& G = it.G;
+  const int nt = it.nbi * it.nbj, wave = static_cast<int>(threadIdx.x >> 6);
+  if (t >= nt) {
+    edge_share<true, false>(it, nt, t, wave, kTile * kTile / 64);
+    return;
+  }
+  const int bi = t / it.nbj, bj = t % it.nbj;
+  const int ti = static_cast<int>(threadIdx.x) / kTile, tj = static_cast<int>(threadIdx.x) % kTile;
   KStep S = it.S;
   S.dtb_pre = gmem(S.dtb_pre);            // null stays null
   const int nbj = it.nbj, nbi = it.nbi;
@@ -338,21 +403,24 @@ __device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int bi, int b
     if (S.dtb_pre) stage_planes<2>(tile, nf, ss, [&](int f) { return S.dtb_pre + f * G.plane; });
     __syncthreads();
   }
-  const int i = i0 + static_cast<int>(threadIdx.y), j = j0 + static_cast<int>(threadIdx.x);
-  if (bi == nbi - 1 && i < 1 + (nbi - 1) * kTile) return;        // done by the tile before
-  if (bj == nbj - 1 && j < it.jlo + (nbj - 1) * kTile) return;
-  if (it.skip && i <= it.sihi && j >= it.sjlo && j <= it.sjhi) return;
-  const TileView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, nf};
-  // phase 1: the geometric auxiliaries of this point, through gaux (own point
-  // only, so no synchronisation); the memory barrier keeps the compiler from
-  // carrying phase-1 values or loads into phase 2, so the two phases do not
-  // add up in registers
-  if (interior_point(G, i, j))
-    rhs_point<false, PHIMODE, true, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-  else
-    rhs_point<false, PHIMODE, false, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
-  asm volatile("" ::: "memory");
-  rhs_point<true, PHIMODE, false, 2>(G, it.P, S, V, gmem(it.yp), gmem(it.acc), gmem(it.yout), gaux, i, j);
+  const int i = i0 + ti, j = j0 + tj;
+  // not the points done by the tile before, outside the item's frame or left
+  // to finebound
+  if (!(bi == nbi - 1 && i < 1 + (nbi - 1) * kTile) && !(bj == nbj - 1 && j < it.jlo + (nbj - 1) * kTile) &&
+      !(it.skip && i <= it.sihi && j >= it.sjlo && j <= it.sjhi) && !finebound_zone(G, it.depth, i, j)) {
+    const TileView V{corner_of(tile, i - ib, j - jb), i - kHalo, j - kHalo, kTileW, kTileSize, nf};
+    // phase 1: the geometric auxiliaries of this point, through gaux (own point
+    // only, so no synchronisation); the memory barrier keeps the compiler from
+    // carrying phase-1 values or loads into phase 2, so the two phases do not
+    // add up in registers
+    if (interior_point(G, i, j))
+      rhs_point<false, PHIMODE, true, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
+    else
+      rhs_point<false, PHIMODE, false, 1>(G, it.P, S, V, nullptr, nullptr, nullptr, gaux, i, j);
+    asm volatile("" ::: "memory");
+    rhs_point<true, PHIMODE, false, 2>(G, it.P, S, V, gmem(it.yp), gmem(it.acc), gmem(it.yout), gaux, i, j);
+  }
+  edge_share<true, false>(it, nt, t, wave, kTile * kTile / 64);
 }
 
 template <bool PHIMODE>
@@ -363,7 +431,7 @@ __global__ void __launch_bounds__(kTile * kTile, 2) k_rhs_phases(const RhsItem* 
                           : static_cast<int>(blockIdx.x);
   const RhsItem& it = find_item(items, n, b);
   const int t = b - it.block0;
-  rhs_phases_tile<PHIMODE>(it, t / it.nbj, t % it.nbj, tile);
+  rhs_phases_tile<PHIMODE>(it, t, tile);
 }
 
 // ------------------------------------------------------ constraints
@@ -474,9 +542,15 @@ __device__ __forceinline__ void finebound_body(const FbItem& it, int blk) {
   const int grp = blk / bpg;
   const long q = static_cast<long>(blk % bpg) * kPtBlock + threadIdx.x;
   if (grp >= finebound_groups(SHIFT, SCALAR) || q >= it.n) return;
-  finebound_point<SHIFT, SCALAR>(it.Gf, it.Gc, it.P, it.T, it.time0, gmem(it.yc), gmem(it.yf), gmem(it.rR0),
-                                 gmem(it.rR1), gmem(it.zL0), gmem(it.zL1), gmem(it.zR0), gmem(it.zR1),
-                                 gmem(it.table)[q], grp);
+  const FbPoint& rec = gmem(it.table)[q];
+  // the strip of time level t0 this point belongs to
+  const double *const r0 = gmem(it.rR0), *const zL0 = gmem(it.zL0), *const zR0 = gmem(it.zR0);
+  const double* const s0 = (rec.which == 0) ? r0 : (rec.which == 1) ? zR0 : zL0;
+  const long sper = static_cast<long>(it.Gf.g) * ((rec.which == 0) ? (it.Gf.Nz + it.Gf.g) : (it.Gf.Nr + it.Gf.g));
+  const long sidx = rec.sidx;
+  finebound_point<SHIFT, SCALAR>(it.Gf, it.Gc, it.P, it.T, it.time0, gmem(it.yc), gmem(it.yf), gmem(it.rR1),
+                                 gmem(it.zL1), gmem(it.zR1), rec, grp,
+                                 [&](int s) { return s0[s * sper + sidx]; });
 }
 
 // restrict: blocks of one field, then the next; one thread per coarse point
@@ -663,6 +737,7 @@ int rhs_tiles(RhsItem* it, bool strips, bool* inner) {
   it->jhi = G.Nz;
   it->skip = 0;
   it->nstr = it->nstz = 0;
+  it->depth = -1;
   if (*inner || strips) {
     const int jlo = G.eqsym ? G.jlo : G.jlo + G.g;
     if (G.Nr - G.g >= kTile && G.Nz - G.g - jlo + 1 >= kTile) {
@@ -714,7 +789,30 @@ void rhs_stencil(const KGrid& G, const KPhys& P, KStencil* W) {
   W->ko_s = P.scalardiss / G.dt * 0.05;
 }
 
-int rhs_blocks(const RhsItem& it) { return it.nbi * it.nbj; }
+int rhs_blocks(const RhsItem& it) { return it.nbi * it.nbj + it.xtra; }
+
+// Blocks of their own for the edge work, only if the whole launch is then
+// resident at once (two blocks per CU): they end before the tiles, whose
+// blocks would take several units each on a small level.  A launch that fills
+// the GPU spreads the units over its tiles' blocks instead, one or two waves
+// of each.  The deeper zone is counted whichever is filled, so that the grid
+// does not depend on whether the clocks meet (a floating comparison).
+void rhs_plan_edges(std::vector<RhsItem>* items, bool shift, bool scalar) {
+  const int waves = (rhs_by_parts(shift, scalar) ? kRhsBlock : kTile * kTile) / 64;
+  auto own = [&](const RhsItem& it) {
+    const int nrt = it.G.Nr + it.G.g, nzt = it.G.Nz + it.G.g;
+    int u = it.E.n > 0 ? finebound_groups(shift, scalar) * static_cast<int>((fb_count(it.G, it.G.g + 2) + 63) / 64) : 0;
+    if (it.E.rR) u += nslots(shift, scalar) * ((it.G.g * (nrt > nzt ? nrt : nzt) + 63) / 64);
+    return (u + waves - 1) / waves;
+  };
+  int total = 0;
+  for (RhsItem& it : *items) {
+    it.xtra = 0;
+    total += rhs_blocks(it) + rhs_strips(it) + own(it);
+  }
+  if (total > kResidentBlocks) return;
+  for (RhsItem& it : *items) it.xtra = own(it);
+}
 int proj_blocks(const ProjItem& it) { return blocks_for(static_cast<long>(it.G.Nr) * (it.G.Nz - it.G.jlo + 1)); }
 int del_blocks(const DelItem& it) { return blocks_for(static_cast<long>(it.G.Nr) * (it.G.Nz - it.G.jlo + 1)); }
 int save_blocks(const SaveItem& it) {
@@ -762,7 +860,7 @@ static int launch_rhs_table_t(const RhsItem* items, int n, int blocks, int strip
   RC_K((rhs_lds<SH, SC, PM>(any_pre, &lds)));
   if constexpr (SH && !SC) {
     (void)strips;
-    hipLaunchKernelGGL((k_rhs_phases<PM>), dim3(blocks), dim3(kTile, kTile, 1), lds, st, items, n, xcd ? 1 : 0);
+    hipLaunchKernelGGL((k_rhs_phases<PM>), dim3(blocks), dim3(kTile * kTile), lds, st, items, n, xcd ? 1 : 0);
     return check_launch();
   } else {
     hipLaunchKernelGGL((k_rhs_table<SH, SC, PM>), dim3(blocks), dim3(kRhsBlock), lds, st, items, n, strips, xcd ? 1 : 0);

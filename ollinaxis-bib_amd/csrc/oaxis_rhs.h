@@ -149,22 +149,6 @@ struct RkUpdate {
   }
 };
 
-// Between two parts of a long expression: no load moves across it, and the
-// partial results given to it are finished before it.  So the stencil values
-// of one part are in registers at a time; left alone, the compiler reads the
-// stencils of every field first and does the arithmetic last, which spills
-// hundreds of registers.
-OA_HD void finish(double& v) {
-#ifdef __HIP_DEVICE_COMPILE__
-  asm volatile("" : "+v"(v));
-#endif
-}
-template <class... T>
-OA_HD void part(T&... v) {
-  (finish(v), ...);
-  asm volatile("" ::: "memory");
-}
-
 // -D'_m g^im of the conformal metric (auxiliary_geometry.f90:1085-1175),
 // differentiated as the products g^ab, like the reference
 template <bool IN, class View>

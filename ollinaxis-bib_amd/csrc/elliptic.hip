@@ -14,8 +14,9 @@
 // Execution: every piece of a coarse step is a kernel whose arguments do not
 // change from step to step -- the level clocks, the time-interpolation
 // coefficients and the finebound depth switch (tp == tl) are formed on the
-// device from clocks kept in device memory -- so one coarse step is captured
-// once as a HIP graph and replayed.  The stopping rule is evaluated on the
+// device from clocks kept in device memory -- so coarse steps are captured
+// once as a HIP graph and replayed (three of them: the states rotate through
+// three planes).  The stopping rule is evaluated on the
 // device at the end of each coarse step; once it fires, every kernel of the
 // later replays returns at once, so the host may run ahead by a whole chunk
 // of steps and reads the outcome after each chunk.
@@ -65,6 +66,7 @@ struct EllCtl {
   // comes after a saveold, and no other kernel reads the clocks.
   int tick[kEllMaxLevels];
   double tick_dt[kEllMaxLevels];
+  unsigned arrived;     // blocks of k_ell_check that have written their partials
 };
 
 // One level's planes for the solve.  u, v: the state at the end of a step
@@ -84,8 +86,10 @@ constexpr int kEllPlanes = 14;
 struct EllLevelArgs {
   KGrid G;
   EllPlanes P;
-  EllClock* clk;
+  EllClock* clk;        // kEllClocks of them: the states and clocks of k_ell_step rotate
+  int cur;              // k_ell_step: the current one
 };
+constexpr int kEllClocks = 3;
 
 __device__ __forceinline__ double pow5(double x) {
   const double x2 = x * x;
@@ -140,9 +144,9 @@ __global__ void __launch_bounds__(kBlk) k_ell_init(KGrid G, EllPlanes E, EllCloc
   if (q < 3 * E.strip_tl) E.strip[q] = 0.0;
 }
 
-__global__ void k_ell_reset(EllCtl* ctl, int stationary, EllClock* clocks, int nlev) {
-  if (threadIdx.x == 0) *ctl = EllCtl{0, 0, stationary, 1.0, 0.0, 0.0, {}, {}};
-  if (static_cast<int>(threadIdx.x) < nlev) clocks[threadIdx.x] = EllClock{0.0, 0.0, 0.0, 0};
+__global__ void k_ell_reset(EllCtl* ctl, int stationary, EllClock* clocks, int nclocks) {
+  if (threadIdx.x == 0) *ctl = EllCtl{0, 0, stationary, 1.0, 0.0, 0.0, {}, {}, 0u};
+  if (static_cast<int>(threadIdx.x) < nclocks) clocks[threadIdx.x] = EllClock{0.0, 0.0, 0.0, 0};
 }
 
 // ------------------------------------------------------------ one step
@@ -154,12 +158,12 @@ __global__ void __launch_bounds__(kBlk) k_ell_saveold(EllLevelArgs a, int fine, 
   if (blockIdx.x == 0 && threadIdx.x == 0)
     for (int l = 0; l < nlev; ++l)
       if (ctl->tick[l]) {                                     // the level clock's step (:997-1004)
-        EllClock c = clocks[l];
+        EllClock c = clocks[kEllClocks * l];
         c.t2 = c.t1;
         c.t1 = c.t;
         c.s = c.s + 1;
         c.t = c.t + ctl->tick_dt[l];
-        clocks[l] = c;
+        clocks[kEllClocks * l] = c;
         ctl->tick[l] = 0;
       }
   const KGrid& G = a.G;
@@ -214,8 +218,41 @@ __device__ __forceinline__ void ell_mark_tick(const EllIterArgs& a, EllCtl* ctl)
   }
 }
 
-// One internal iteration of one level (:691-915): sources of u and v, the
-// Kreiss-Oliger terms on v, the radiative boundary of v, the RK4
+// Sources of u and v at a point (:691-893): the flat Laplacian, the
+// coefficients, the damping, the Kreiss-Oliger terms on v and the radiative
+// boundary of v.  U, V: the iteration's input; s1, s5: the coefficients at
+// the point (s5 read only when it matters).
+template <class F, class S5>
+__device__ __forceinline__ void ell_sources(const KGrid& G, const F& U, const F& V, double s1, const S5& s5, double eta,
+                                            double diss, double idt, int i, int j, double& su, double& sv) {
+  const double r = coord_r(G, i), z = coord_z(G, j);
+  const double u = U(i, j), v = V(i, j);
+  su = v;
+  // flat Laplacian, the coefficients and the damping (:791-851)
+  const double Dr_u = s_d1r(U, G, i, j), Drr_u = s_d2r(U, G, i, j), Dzz_u = s_d2z(U, G, i, j);
+  sv = Drr_u + Dzz_u + Dr_u / r;
+  // S0 is zero for every supported initial data (subtracting +0 changes
+  // nothing) and S5 without a scalar potential (adding a zero changes the
+  // value of nothing either): their planes are read only when they matter
+  sv = sv + s1 * u;
+  sv = s5(sv, u);
+  sv = sv - eta * v;
+  // dissipation on v (dissipation.f90:181-199): rho terms for i <= Nr-3,
+  // z terms for 1 <= j <= Nz-3
+  if (i <= G.Nr - 3)
+    sv = sv - diss * idt * (20.0 * V(i, j) - 15.0 * (V(i + 1, j) + V(i - 1, j)) + 6.0 * (V(i + 2, j) + V(i - 2, j))
+                            - (V(i + 3, j) + V(i - 3, j))) / 20.0;
+  if (j >= 1 && j <= G.Nz - 3)
+    sv = sv - diss * idt * (20.0 * V(i, j) - 15.0 * (V(i, j + 1) + V(i, j - 1)) + 6.0 * (V(i, j + 2) + V(i, j - 2))
+                            - (V(i, j + 3) + V(i, j - 3))) / 20.0;
+  // radiative boundary on v with v = 1, v0 = 0 (radbound.f90:44-70)
+  if (i == G.Nr || j == G.Nz || (!G.eqsym && j == 1 - G.g)) {
+    const double rr = sqrt(fma(z, z, r * r));
+    sv = -1.0 * (r * s_d1r(V, G, i, j) + z * s_d1z(V, G, i, j) + (v - 0.0)) / rr;
+  }
+}
+
+// One internal iteration of one level (:691-915): the sources, the RK4
 // accumulators and the update, at every computed point with its parity
 // images (both fields are even on the axis and the equator).
 __device__ __forceinline__ void ell_iter_point(const EllIterArgs& a, int i, int j) {
@@ -223,31 +260,9 @@ __device__ __forceinline__ void ell_iter_point(const EllIterArgs& a, int i, int 
   const EllPlanes& E = a.L.P;
   const long k = IDX(G, i, j);
   const Plane U{a.uin, G}, V{a.vin, G};
-  const double r = coord_r(G, i), z = coord_z(G, j);
-  const double u = U(i, j), v = V(i, j);
-  double su = v;
-  // flat Laplacian, the coefficients and the damping (:791-851)
-  const double Dr_u = s_d1r(U, G, i, j), Drr_u = s_d2r(U, G, i, j), Dzz_u = s_d2z(U, G, i, j);
-  double sv = Drr_u + Dzz_u + Dr_u / r;
-  // S0 is zero for every supported initial data (subtracting +0 changes
-  // nothing) and S5 without a scalar potential (adding a zero changes the
-  // value of nothing either): their planes are read only when they matter
-  sv = sv + E.s1[k] * u;
-  if (a.s5) sv = sv + E.s5[k] * pow5(u);
-  sv = sv - a.eta * v;
-  // dissipation on v (dissipation.f90:181-199): rho terms for i <= Nr-3,
-  // z terms for 1 <= j <= Nz-3
-  if (i <= G.Nr - 3)
-    sv = sv - a.diss * a.idt * (20.0 * V(i, j) - 15.0 * (V(i + 1, j) + V(i - 1, j)) + 6.0 * (V(i + 2, j) + V(i - 2, j))
-                                - (V(i + 3, j) + V(i - 3, j))) / 20.0;
-  if (j >= 1 && j <= G.Nz - 3)
-    sv = sv - a.diss * a.idt * (20.0 * V(i, j) - 15.0 * (V(i, j + 1) + V(i, j - 1)) + 6.0 * (V(i, j + 2) + V(i, j - 2))
-                                - (V(i, j + 3) + V(i, j - 3))) / 20.0;
-  // radiative boundary on v with v = 1, v0 = 0 (radbound.f90:44-70)
-  if (i == G.Nr || j == G.Nz || (!G.eqsym && j == 1 - G.g)) {
-    const double rr = sqrt(r * r + z * z);
-    sv = -1.0 * (r * s_d1r(V, G, i, j) + z * s_d1z(V, G, i, j) + (v - 0.0)) / rr;
-  }
+  double su, sv;
+  ell_sources(G, U, V, E.s1[k], [&](double s, double u) { return a.s5 ? s + E.s5[k] * pow5(u) : s; }, a.eta, a.diss,
+              a.idt, i, j, su, sv);
   // RK4 accumulators (:895-907)
   if (a.rk4) {
     if (a.iter == 1) {
@@ -355,6 +370,221 @@ __global__ void __launch_bounds__(kBlk) k_ell_iter_fb(EllStepArgs a, EllCtl* ctl
 }
 
 
+// ------------------------------------------------ a whole ICN step of a level
+// saveold, the three ICN iterations and their finebounds as one launch.  A
+// block owns 16 x 16 points and stages u, v and S1 of the 34 x 34 points
+// around them; each iteration needs 3 points more on every side than the next
+// (the dissipation's reach), so it runs the iterations on 28 x 28, 22 x 22 and
+// 16 x 16 points in LDS, twice the arithmetic of the three launches, and only
+// the last one leaves the block.  Bound by latency: a level step of 128 x 256
+// took a copy of 4 us and three launches of 6 us, each mostly its start and
+// one round trip to memory.  With it the solve of a pulse on two such levels
+// went from 233 to 110 ms, a Brill wave's on five levels of 256 x 512 from 3.3
+// to 2.1 s.  The states rotate through three planes instead
+// of being copied: a step reads the current one, finebound also reads the one
+// before at its own zone (time level t-1; no strips), and the result goes to
+// the third.  The level's clock rotates with them.
+constexpr int kEsTile = 16, kEsHalo = 9, kEsW = kEsTile + 2 * kEsHalo, kEsSize = kEsW * kEsW, kEsBlock = 512;
+constexpr int kEsZone = 2;         // zone points per thread, at most (540 in a block)
+
+struct EllStep1Args {
+  KGrid G, Gc;
+  const double *u0, *v0;             // state at the start of the step
+  const double *um, *vm;             // state at the start of the step before
+  double *u1, *v1;                   // state at its end
+  const double *s1, *s5;
+  double* sv;                        // base level: the last source of v
+  double eta, diss, idt;
+  int use5, base;
+  int nbj;
+  const double *uc, *vc;             // coarse state (already advanced)
+  const FbPoint* tab[2];             // zones of depth g+2 (tp == tl) and g-1
+  const EllClock* cclk;              // coarse clock; null on the base level
+  const EllClock* clk;               // this level's clock, and where the step leaves it
+  EllClock* next;
+};
+
+// the record of zone point (i, j) in the table of depth D (fb_geometry's order)
+__device__ __forceinline__ long ell_zone_record(const KGrid& G, int D, int i, int j) {
+  const int g = G.g, nrt = G.Nr + g, nzt = G.Nz + g;
+  const long n_r = static_cast<long>(D + 1) * nzt;
+  if (j >= G.Nz - D) return n_r + static_cast<long>(G.Nz - j) * nrt + (i + g - 1);
+  if (!G.eqsym && j <= 1 - g + D) return n_r + static_cast<long>(D + 1 + j - (1 - g)) * nrt + (i + g - 1);
+  return static_cast<long>(G.Nr - i) * nzt + (j + g - 1);
+}
+
+__device__ __forceinline__ bool ell_in_zone(const KGrid& G, int D, int i, int j) {
+  return i >= G.Nr - D || j >= G.Nz - D || (!G.eqsym && j <= 1 - G.g + D);
+}
+
+struct EsPlane {                     // a staged plane
+  const double* p;
+  int ei, ej;
+  __device__ __forceinline__ double operator()(int i, int j) const { return p[(i - ei) * kEsW + (j - ej)]; }
+};
+
+__global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl* ctl) {
+  if (ctl->done) return;
+  __shared__ double st[6][kEsSize];  // u, v: start, first and second iteration
+  __shared__ double sS1[kEsSize];
+  const KGrid& G = a.G;
+  const int g = G.g, t = static_cast<int>(threadIdx.x);
+  const int bi = static_cast<int>(blockIdx.x) / a.nbj, bj = static_cast<int>(blockIdx.x) % a.nbj;
+  // the last tiles end at the level's edge (and overlap the ones before, with
+  // the same values): the one-sided stencils there reach 5 points inwards,
+  // more than the 3 of an iteration's halo
+  const int i0 = max(min(1 + bi * kEsTile, G.Nr - kEsTile + 1), 1);
+  const int j0 = max(min(G.jlo + bj * kEsTile, G.Nz - kEsTile + 1), G.jlo);
+  const int ei = i0 - kEsHalo, ej = j0 - kEsHalo;
+  if (blockIdx.x == 0 && t == 0) {                                    // :997-1004
+    EllClock c = *a.clk;
+    c.t2 = c.t1;
+    c.t1 = c.t;
+    c.s = c.s + 1;
+    c.t = c.t + G.dt;
+    *a.next = c;
+  }
+#pragma unroll
+  for (int q0 = 0; q0 < kEsSize; q0 += kEsBlock) {
+    const int q = q0 + t;
+    if (q < kEsSize) {
+      const int i = min(max(ei + q / kEsW, 1 - g), G.Nr), j = min(max(ej + q % kEsW, 1 - g), G.Nz);
+      const long k = IDX(G, i, j);
+      st[0][q] = a.u0[k];
+      st[1][q] = a.v0[k];
+      sS1[q] = a.s1[k];
+    }
+  }
+  // the fine-boundary zone (depth g+2) among the staged points: rows i >= Nr -
+  // D, then the columns of the rest; the coarse level's interpolants for both
+  // depths, which no iteration changes
+  const bool fine = a.cclk != nullptr;
+  double tp = 0.0, ct0 = 0.0, tm1 = 0.0;
+  int zr = 0, zi = 0, zl = 0, zh = 0, nz = 0;   // rows of the rho strip and of the rest; columns low, high
+  const int hi_i = min(i0 + kEsTile - 1 + 6, G.Nr), lo_i = max(i0 - 6, 1);
+  const int hi_j = min(j0 + kEsTile - 1 + 6, G.Nz), lo_j = max(j0 - 6, G.jlo);
+  const int wj = hi_j - lo_j + 1;
+  if (fine) {
+    tp = a.cclk->t;
+    ct0 = a.clk->t;
+    tm1 = a.clk->t1;
+    const int D = g + 2;
+    zr = max(0, hi_i - max(lo_i, G.Nr - D) + 1);
+    zi = hi_i - lo_i + 1 - zr;
+    zh = max(0, hi_j - max(lo_j, G.Nz - D) + 1);
+    zl = G.eqsym ? 0 : max(0, min(hi_j, 1 - g + D) - lo_j + 1);
+    if (zl + zh > wj) { zl = wj; zh = 0; }
+    nz = zr * wj + zi * (zl + zh);
+  }
+  auto zone_point = [&](int q, int& i, int& j) {
+    if (q < zr * wj) {
+      i = hi_i - q / wj;
+      j = lo_j + q % wj;
+    } else {
+      const int q2 = q - zr * wj, w = zl + zh, c = q2 % w;
+      i = lo_i + q2 / w;
+      j = c < zl ? lo_j + c : hi_j - (c - zl);
+    }
+  };
+  const bool same3 = fine && tp == ct0 + G.dt, same12 = fine && tp == ct0 + 0.5 * G.dt;
+  double zu[kEsZone][2], zv[kEsZone][2], mu[kEsZone], mv[kEsZone];   // [.][0]: depth g+2, [.][1]: g-1
+  if (fine && nz > 0) {
+#pragma unroll
+    for (int z = 0; z < kEsZone; ++z) {
+      const int q = t + z * kEsBlock;
+      mu[z] = mv[z] = 0.0;
+      zu[z][0] = zu[z][1] = zv[z][0] = zv[z][1] = 0.0;
+      if (q >= nz) continue;
+      int i, j;
+      zone_point(q, i, j);
+      if (same3 || same12) {
+        const Cell c = a.tab[0][ell_zone_record(G, g + 2, i, j)].c;
+        zu[z][0] = apply(c, a.uc, a.Gc);
+        zv[z][0] = apply(c, a.vc, a.Gc);
+      }
+      if (!(same3 && same12) && ell_in_zone(G, g - 1, i, j)) {
+        const Cell c = a.tab[1][ell_zone_record(G, g - 1, i, j)].c;
+        zu[z][1] = apply(c, a.uc, a.Gc);
+        zv[z][1] = apply(c, a.vc, a.Gc);
+      }
+      if (ell_in_zone(G, g - 1, i, j)) {        // inside the strips of the saved time levels
+        const long k = IDX(G, i, j);
+        mu[z] = a.um[k];
+        mv[z] = a.vm[k];
+      }
+    }
+  }
+  __syncthreads();
+  const EsPlane U0{st[0], ei, ej}, V0{st[1], ei, ej};
+#pragma unroll
+  for (int k = 1; k <= 3; ++k) {
+    const double dtw = (k < 3) ? 0.5 * G.dt : G.dt;
+    const EsPlane U{st[2 * (k - 1)], ei, ej}, V{st[2 * (k - 1) + 1], ei, ej};
+    double* const ou = st[k < 3 ? 2 * k : 0];   // unused on the last iteration
+    double* const ov = st[k < 3 ? 2 * k + 1 : 1];
+    const int R = 3 * (3 - k), W = kEsTile + 2 * R;
+    const double tl = ct0 + dtw;
+    const bool same = fine && tp == tl;
+    const int D = same ? g + 2 : g - 1;
+    // a value at (i, j): into the block's plane with its images, or the level
+    auto keep = [&](int i, int j, double nu, double nv) {
+      if (k == 3) {
+        put(a.u1, G, i, j, nu, 1.0, 1.0);
+        put(a.v1, G, i, j, nv, 1.0, 1.0);
+        return;
+      }
+      auto set = [&](int ii, int jj) {
+        const int x = ii - ei, y = jj - ej;
+        if (x < 0 || x >= kEsW || y < 0 || y >= kEsW) return;
+        ou[x * kEsW + y] = nu;
+        ov[x * kEsW + y] = nv;
+      };
+      set(i, j);
+      if (i <= g) set(1 - i, j);
+      if (G.eqsym && j >= 1 && j <= g) {
+        set(i, 1 - j);
+        if (i <= g) set(1 - i, 1 - j);
+      }
+    };
+    for (int q = t; q < W * W; q += kEsBlock) {
+      const int i = i0 - R + q / W, j = j0 - R + q % W;
+      if (i < 1 || i > G.Nr || j < G.jlo || j > G.Nz) continue;
+      if (fine && ell_in_zone(G, D, i, j)) continue;
+      double su, sv;
+      const long kk = IDX(G, i, j);
+      ell_sources(G, U, V, sS1[(i - ei) * kEsW + (j - ej)],
+                  [&](double s, double u) { return a.use5 ? s + a.s5[kk] * pow5(u) : s; }, a.eta, a.diss, a.idt, i, j,
+                  su, sv);
+      keep(i, j, U0(i, j) + dtw * su, V0(i, j) + dtw * sv);
+      if (k == 3 && a.base) a.sv[kk] = sv;
+    }
+    if (fine && nz > 0) {
+      // finebound (finebound.f90:70-400), as ell_fb_point forms it
+#pragma unroll
+      for (int z = 0; z < kEsZone; ++z) {
+        const int q = t + z * kEsBlock;
+        if (q >= nz) continue;
+        int i, j;
+        zone_point(q, i, j);
+        if (i < i0 - R || i >= i0 + kEsTile + R || j < j0 - R || j >= j0 + kEsTile + R) continue;
+        if (!ell_in_zone(G, D, i, j)) continue;
+        const double t0 = ct0;
+        const bool inside = ell_in_zone(G, g - 1, i, j);
+        const double au = zu[z][same ? 0 : 1], av = zv[z][same ? 0 : 1];
+        auto in_time = [&](double aux2, double start, double before) {
+          if (tm1 == 0.0) return (tl - t0) / (tp - t0) * aux2 + (tl - tp) / (t0 - tp) * start;
+          const double b0 = inside ? start : 0.0, b1 = before;
+          return (tl - t0) * (tl - tm1) / ((tp - t0) * (tp - tm1)) * aux2 +
+                 (tl - tp) * (tl - tm1) / ((t0 - tp) * (t0 - tm1)) * b0 +
+                 (tl - tp) * (tl - t0) / ((tm1 - tp) * (tm1 - t0)) * b1;
+        };
+        keep(i, j, in_time(au, U0(i, j), mu[z]), in_time(av, V0(i, j), mv[z]));
+      }
+    }
+    if (k < 3) __syncthreads();
+  }
+}
+
 struct EllRsArgs {
   KGrid Gf, Gc;
   const double* uf; const double* vf;
@@ -367,11 +597,7 @@ struct EllRsArgs {
 // images, the coarse level's symmetries that wavestep applies right after
 // it (:1136-1149) as images of each written point (the SOR solve applies
 // none)
-__global__ void __launch_bounds__(kBlk) k_ell_restrict(EllRsArgs a, const EllCtl* __restrict__ ctl) {
-  if (ctl->done) return;
-  const long q = static_cast<long>(blockIdx.x) * kBlk + threadIdx.x;
-  if (q >= static_cast<long>(a.nic) * a.njc) return;
-  const int ic = a.ic0 + static_cast<int>(q / a.njc), jc = a.jc0 + static_cast<int>(q % a.njc);
+__device__ __forceinline__ void ell_restrict_point(const EllRsArgs& a, int ic, int jc) {
   const KGrid& Gf = a.Gf;
   const KGrid& Gc = a.Gc;
   const int g = Gc.g;
@@ -394,72 +620,98 @@ __global__ void __launch_bounds__(kBlk) k_ell_restrict(EllRsArgs a, const EllCtl
   }
 }
 
-// Residual and change of the base level after a coarse step, per block:
-// sum of sv^2 (i in [1, Nr-g], j in [1, Nz-g], wave_elliptic.f90:321-341),
-// max |u - up| and max |u| over the same range.
-__global__ void __launch_bounds__(kBlk) k_ell_check(KGrid G, EllPlanes E, double* __restrict__ part,
-                                                    const EllCtl* __restrict__ ctl) {
+__global__ void __launch_bounds__(kBlk) k_ell_restrict(EllRsArgs a, const EllCtl* __restrict__ ctl) {
+  if (ctl->done) return;
+  const long q = static_cast<long>(blockIdx.x) * kBlk + threadIdx.x;
+  if (q >= static_cast<long>(a.nic) * a.njc) return;
+  ell_restrict_point(a, a.ic0 + static_cast<int>(q / a.njc), a.jc0 + static_cast<int>(q % a.njc));
+}
+
+// Residual and change of the base level after a coarse step, per block: sum
+// of sv^2 (i in [1, Nr-g], j in [1, Nz-g], wave_elliptic.f90:321-341), max |u
+// - up| and max |u| over the same range.  The last block to arrive combines
+// the blocks' partials in block order and applies the stopping rule.
+// Reference (:303): continue while step < 100 or (gres > WE_epsilon and step <
+// WE_maxiter) -- a NaN residual stops.  Stationary rule (all-levels phase
+// only, when enabled): stop once the window maximum over 100 steps of max|u -
+// up| / max|u| is at most 1e-12 and above half the previous window's.
+struct EllCheckArgs {
+  KGrid G;
+  const double *sv, *u, *up;
+  double* part;
+  double nntot, eps;
+  int maxiter;
+};
+constexpr int kEllParts = 256;
+static_assert(kEllParts == kBlk, "one partial per thread of the last block");
+
+__global__ void __launch_bounds__(kBlk) k_ell_check(EllCheckArgs a, EllCtl* ctl) {
   if (ctl->done) return;
   __shared__ double ssq[kBlk], sdu[kBlk], smu[kBlk];
+  __shared__ unsigned last;
+  const KGrid& G = a.G;
   const int ni = G.Nr - G.g, nj = G.Nz - G.g;
   const long n = static_cast<long>(ni) * nj;
   double sq = 0.0, du = 0.0, mu = 0.0;
   for (long q = static_cast<long>(blockIdx.x) * kBlk + threadIdx.x; q < n; q += static_cast<long>(gridDim.x) * kBlk) {
     const int i = 1 + static_cast<int>(q / nj), j = 1 + static_cast<int>(q % nj);
     const long k = IDX(G, i, j);
-    const double s = E.sv[k];
+    const double s = a.sv[k];
     sq += s * s;
-    du = fmax(du, fabs(E.u[k] - E.up[k]));
-    mu = fmax(mu, fabs(E.u[k]));
+    du = fmax(du, fabs(a.u[k] - a.up[k]));
+    mu = fmax(mu, fabs(a.u[k]));
   }
   const int t = static_cast<int>(threadIdx.x);
+  auto tree = [&](bool sum) {
+    for (int h = kBlk / 2; h > 0; h >>= 1) {
+      if (t < h) {
+        if (sum) ssq[t] += ssq[t + h];
+        sdu[t] = fmax(sdu[t], sdu[t + h]);
+        smu[t] = fmax(smu[t], smu[t + h]);
+      }
+      __syncthreads();
+    }
+  };
   ssq[t] = sq; sdu[t] = du; smu[t] = mu;
   __syncthreads();
-  for (int h = kBlk / 2; h > 0; h >>= 1) {
-    if (t < h) {
-      ssq[t] += ssq[t + h];
-      sdu[t] = fmax(sdu[t], sdu[t + h]);
-      smu[t] = fmax(smu[t], smu[t + h]);
-    }
-    __syncthreads();
-  }
+  tree(true);
   if (t == 0) {
-    part[3 * blockIdx.x] = ssq[0];
-    part[3 * blockIdx.x + 1] = sdu[0];
-    part[3 * blockIdx.x + 2] = smu[0];
+    a.part[3 * blockIdx.x] = ssq[0];
+    a.part[3 * blockIdx.x + 1] = sdu[0];
+    a.part[3 * blockIdx.x + 2] = smu[0];
+    __threadfence();
+    last = atomicAdd(&ctl->arrived, 1u);
   }
-}
-
-// The stopping rule after a coarse step.  Reference (:303): continue while
-// step < 100 or (gres > WE_epsilon and step < WE_maxiter) -- a NaN residual
-// stops.  Stationary rule (all-levels phase only, when enabled): stop once
-// the window maximum over 100 steps of max|u - up| / max|u| is at most
-// 1e-12 and above half the previous window's.
-__global__ void k_ell_decide(int nparts, const double* __restrict__ part, double nntot, double eps, int maxiter,
-                             EllCtl* ctl) {
-  if (threadIdx.x != 0 || ctl->done) return;
-  double sq = 0.0, du = 0.0, mu = 0.0;
-  for (int b = 0; b < nparts; ++b) {
-    sq += part[3 * b];
-    du = fmax(du, part[3 * b + 1]);
-    mu = fmax(mu, part[3 * b + 2]);
-  }
-  EllCtl c = *ctl;
-  c.step += 1;
-  c.gres = sqrt(sq / nntot);
-  const bool more = (c.step < 100) || (c.gres > eps && c.step < maxiter);
+  __syncthreads();
+  if (last != gridDim.x - 1) return;
+  __threadfence();
+  ssq[t] = a.part[3 * t];
+  sdu[t] = a.part[3 * t + 1];
+  smu[t] = a.part[3 * t + 2];
+  __syncthreads();
+  tree(false);
+  if (t != 0) return;
+  double total = 0.0;
+#pragma unroll 16
+  for (int b = 0; b < kEllParts; ++b) total += ssq[b];
+  EllCtl& c = *ctl;
+  c.arrived = 0u;
+  const int step = c.step + 1;
+  const double gres = sqrt(total / a.nntot);
+  const bool more = (step < 100) || (gres > a.eps && step < a.maxiter);
   int done = more ? 0 : 1;
   if (!done && c.stationary) {
-    const double rel = du / mu;
+    const double rel = sdu[0] / smu[0];
     if (rel > c.wmax) c.wmax = rel;
-    if (c.step % 100 == 0) {
+    if (step % 100 == 0) {
       if (c.wmax <= 1.0e-12 && c.wmax > 0.5 * c.wprev) done = 1;
       c.wprev = c.wmax;
       c.wmax = 0.0;
     }
   }
+  c.step = step;
+  c.gres = gres;
   c.done = done;
-  *ctl = c;
 }
 
 // interpolate the base-level solution onto every point of a finer level
@@ -746,9 +998,9 @@ struct EllSolver {
       const long per_f = static_cast<long>(G.g) * (G.Nz + G.g) + 2L * G.g * (G.Nr + G.g);
       total += 3 * 2 * static_cast<size_t>(per_f);
     }
-    nparts = 256;
+    nparts = kEllParts;
     const size_t ctl_doubles = (sizeof(EllCtl) + sizeof(double) - 1) / sizeof(double);
-    const size_t clk_doubles = (sizeof(EllClock) * nlev + sizeof(double) - 1) / sizeof(double);
+    const size_t clk_doubles = (sizeof(EllClock) * kEllClocks * nlev + sizeof(double) - 1) / sizeof(double);
     const size_t sctl_doubles = (sizeof(SorCtl) + sizeof(double) - 1) / sizeof(double);
     const size_t bytes = sizeof(double) * (total + 3 * nparts + ctl_doubles + clk_doubles + sctl_doubles);
     ELLHIP(hipMalloc(&arena, bytes), "device allocation");
@@ -770,7 +1022,8 @@ struct EllSolver {
       for (int k = 0; k < kEllPlanes; ++k) *planes[k] = b + k * pl;
       a.P.strip = arena + strip_off[l];
       a.P.strip_tl = 2 * (static_cast<long>(a.G.g) * (a.G.Nz + a.G.g) + 2L * a.G.g * (a.G.Nr + a.G.g));
-      a.clk = clocks + l;
+      a.clk = clocks + kEllClocks * l;
+      a.cur = 0;
     }
     return OA_OK;
   }
@@ -792,8 +1045,87 @@ struct EllSolver {
     return OA_OK;
   }
 
+  // The reference's default relaxation, ICN with three iterations, takes a
+  // level step as one launch (k_ell_step); RK4 and other iteration counts
+  // need another halo and accumulators, and go iteration by iteration.
+  bool one_launch() const { return h->p.WE_method != OA_RK4 && h->p.icniter == 3; }
+
+  // the planes the state rotates through (k_ell_step); iteration by
+  // iteration it stays in the first
+  double* u_of(const EllLevelArgs& a, int k) const { return k == 0 ? a.P.u : k == 1 ? a.P.up : a.P.t1u; }
+  double* v_of(const EllLevelArgs& a, int k) const { return k == 0 ? a.P.v : k == 1 ? a.P.vp : a.P.t1v; }
+  double* u_now(const EllLevelArgs& a) const { return u_of(a, a.cur); }
+  double* v_now(const EllLevelArgs& a) const { return v_of(a, a.cur); }
+
+  int icn_step(int level) {
+    const oa_params& p = h->p;
+    EllLevelArgs& a = lev[level];
+    const int cur = a.cur, nxt = (cur + 1) % 3, old = (cur + 2) % 3;
+    EllStep1Args s{};
+    s.G = a.G;
+    s.u0 = u_of(a, cur);
+    s.v0 = v_of(a, cur);
+    s.um = u_of(a, old);
+    s.vm = v_of(a, old);
+    s.u1 = u_of(a, nxt);
+    s.v1 = v_of(a, nxt);
+    s.s1 = a.P.s1;
+    s.s5 = a.P.s5;
+    s.sv = a.P.sv;
+    s.eta = p.WE_eta;
+    s.diss = p.WE_diss;
+    s.idt = 1.0 / a.G.dt;
+    s.use5 = (p.idata == OA_IDATA_SCALARPULSE && p.scalarpotential != OA_POT_NONE) ? 1 : 0;
+    s.base = (level == 0) ? 1 : 0;
+    s.nbj = (a.G.Nz - a.G.jlo + kEsTile) / kEsTile;
+    s.clk = a.clk + cur;
+    s.next = a.clk + nxt;
+    if (level > 0) {
+      const EllLevelArgs& c = lev[level - 1];
+      s.Gc = c.G;
+      s.uc = u_now(c);
+      s.vc = v_now(c);
+      s.tab[0] = h->L[level].fbtab[0];
+      s.tab[1] = h->L[level].fbtab[1];
+      s.cclk = c.clk + c.cur;
+    }
+    const int nbi = (a.G.Nr + kEsTile - 1) / kEsTile;
+    hipLaunchKernelGGL(k_ell_step, dim3(nbi * s.nbj), dim3(kEsBlock), 0, st, s, ctl);
+    ELLRC(launched("ICN step"));
+    a.cur = nxt;
+    return OA_OK;
+  }
+
   // wavestep(level) as launches (recursion into the levels up to nlmax)
   int wavestep(int level, int nlmax) {
+    if (one_launch()) ELLRC(icn_step(level));
+    else ELLRC(iterations(level));
+    if (level < nlmax) {
+      ELLRC(wavestep(level + 1, nlmax));
+      ELLRC(wavestep(level + 1, nlmax));
+      // the second step of level+1 brings its clock to an even step count:
+      // restrict onto this level (:1106-1157)
+      const EllLevelArgs& a = lev[level];
+      const EllLevelArgs& f = lev[level + 1];
+      EllRsArgs rs{};
+      rs.Gf = f.G;
+      rs.Gc = a.G;
+      rs.uf = u_now(f);
+      rs.vf = v_now(f);
+      rs.uc = u_now(a);
+      rs.vc = v_now(a);
+      rs.interporder = h->p.interporder;
+      rs.images = 1;
+      restrict_box(f.G, a.G, &rs.ic0, &rs.nic, &rs.jc0, &rs.njc);
+      hipLaunchKernelGGL(k_ell_restrict, dim3(blocks(static_cast<long>(rs.nic) * rs.njc)), dim3(kBlk), 0, st, rs,
+                         ctl);
+      ELLRC(launched("restrict"));
+    }
+    return OA_OK;
+  }
+
+  // saveold and the internal iterations of one level's step
+  int iterations(int level) {
     const oa_params& p = h->p;
     EllLevelArgs& a = lev[level];
     const KGrid& G = a.G;
@@ -874,53 +1206,44 @@ struct EllSolver {
         ELLRC(launched("iteration and finebound"));
       }
     }
-    if (level < nlmax) {
-      ELLRC(wavestep(level + 1, nlmax));
-      ELLRC(wavestep(level + 1, nlmax));
-      // the second step of level+1 brings its clock to an even step count:
-      // restrict onto this level (:1106-1157)
-      const EllLevelArgs& f = lev[level + 1];
-      EllRsArgs rs{};
-      rs.Gf = f.G;
-      rs.Gc = G;
-      rs.uf = f.P.u;
-      rs.vf = f.P.v;
-      rs.uc = a.P.u;
-      rs.vc = a.P.v;
-      rs.interporder = p.interporder;
-      rs.images = 1;
-      restrict_box(f.G, G, &rs.ic0, &rs.nic, &rs.jc0, &rs.njc);
-      hipLaunchKernelGGL(k_ell_restrict, dim3(blocks(static_cast<long>(rs.nic) * rs.njc)), dim3(kBlk), 0, st, rs,
-                         ctl);
-      ELLRC(launched("restrict"));
-    }
     return OA_OK;
   }
 
   int coarse_step(int nlmax) {
     ELLRC(wavestep(0, nlmax));
     const EllLevelArgs& b = lev[0];
-    hipLaunchKernelGGL(k_ell_check, dim3(nparts), dim3(kBlk), 0, st, b.G, b.P, part, ctl);
-    ELLRC(launched("residual"));
-    const double nntot = static_cast<double>(b.G.Nr) * static_cast<double>(b.G.Nz);
-    hipLaunchKernelGGL(k_ell_decide, dim3(1), dim3(64), 0, st, nparts, part, nntot, h->p.WE_epsilon,
-                       h->p.WE_maxiter, ctl);
-    return launched("stopping rule");
+    EllCheckArgs c{};
+    c.G = b.G;
+    c.sv = b.P.sv;
+    c.u = u_now(b);
+    c.up = one_launch() ? u_of(b, (b.cur + 2) % 3) : b.P.up;
+    c.part = part;
+    c.nntot = static_cast<double>(b.G.Nr) * static_cast<double>(b.G.Nz);
+    c.eps = h->p.WE_epsilon;
+    c.maxiter = h->p.WE_maxiter;
+    hipLaunchKernelGGL(k_ell_check, dim3(nparts), dim3(kBlk), 0, st, c, ctl);
+    return launched("residual and stopping rule");
   }
 
-  // one phase: coarse steps over levels 0..nlmax until the rule fires.  The
-  // coarse step is captured once as a graph and replayed, unless the handle's
+  // one phase: coarse steps over levels 0..nlmax until the rule fires.  Three
+  // coarse steps, after which every rotation is back where it was, are
+  // captured once as a graph and replayed, unless the handle's
   // caller turned graphs off (oa_set_graphs): then every step is launched
   // kernel by kernel, with the same kernels in the same order.
   int phase(int nlmax, int stationary_rule, int* steps, double* gres) {
-    hipLaunchKernelGGL(k_ell_reset, dim3(1), dim3(64), 0, st, ctl, stationary_rule, clocks, nlev);
+    hipLaunchKernelGGL(k_ell_reset, dim3(1), dim3(64), 0, st, ctl, stationary_rule, clocks, kEllClocks * nlev);
     ELLRC(launched("reset"));
     const bool use_graph = h->plan.graphs || h->plan.tuner.enabled;
+    constexpr int kPerGraph = 3;
+    const std::vector<EllLevelArgs> start = lev;
+    // k_ell_reset starts the first clock of each level, and the planes before
+    // the first step are never read (tm1 = 0)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     if (use_graph) {
       ELLHIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "graph capture");
-      const int rc = coarse_step(nlmax);
+      int rc = OA_OK;
+      for (int k = 0; rc == OA_OK && k < kPerGraph; ++k) rc = coarse_step(nlmax);
       hipGraph_t captured = nullptr;
       const hipError_t ec = hipStreamEndCapture(st, &captured);
       if (rc != OA_OK) {
@@ -939,9 +1262,9 @@ struct EllSolver {
     const int maxiter = h->p.WE_maxiter;
     long launched_steps = 0;
     for (;;) {
-      // at least 100 steps are always taken; then chunks of 64
-      const int chunk = (launched_steps == 0) ? 100 : 64;
-      for (int k = 0; k < chunk && status == OA_OK; ++k) {
+      // at least 100 steps are always taken; then chunks of 66
+      const int chunk = (launched_steps == 0) ? 102 : 66;
+      for (int k = 0; k < chunk && status == OA_OK; k += use_graph ? kPerGraph : 1) {
         if (!use_graph) {
           status = coarse_step(nlmax);
           continue;
@@ -973,6 +1296,12 @@ struct EllSolver {
     if (status != OA_OK) return status;
     *steps = host_ctl->step;
     *gres = host_ctl->gres;
+    // where the steps taken left the rotation (later launches did nothing)
+    if (one_launch())
+      for (int l = 0; l < nlev; ++l) {
+        const long taken = l <= nlmax ? static_cast<long>(host_ctl->step) << l : 0;
+        lev[l].cur = static_cast<int>((start[l].cur + taken) % 3);
+      }
     return OA_OK;
   }
 
@@ -1087,7 +1416,7 @@ struct EllSolver {
       *steps1 += it;
     }
     // k_ell_restrict runs while the wave solve's control block says not done
-    hipLaunchKernelGGL(k_ell_reset, dim3(1), dim3(64), 0, st, ctl, 0, clocks, nlev);
+    hipLaunchKernelGGL(k_ell_reset, dim3(1), dim3(64), 0, st, ctl, 0, clocks, kEllClocks * nlev);
     ELLRC(launched("reset"));
     for (int l = 1; l < nlev; ++l) {
       const EllLevelArgs& f = lev[l];
@@ -1117,12 +1446,12 @@ struct EllSolver {
     ELLRC(phase(nlmax_old > 0 ? 0 : nlmax_old, 0, steps0, gres));
     if (nlmax_old > 0 && *steps0 != h->p.ELL_maxiter) {
       const EllLevelArgs& b = lev[0];
-      hipLaunchKernelGGL(k_ell_zero, dim3(blocks(b.G.plane)), dim3(kBlk), 0, st, b.G.plane, b.P.v);
+      hipLaunchKernelGGL(k_ell_zero, dim3(blocks(b.G.plane)), dim3(kBlk), 0, st, b.G.plane, v_now(b));
       ELLRC(launched("v = 0"));
       for (int l = 1; l <= nlmax_old; ++l) {
         const EllLevelArgs& f = lev[l];
         const long n = static_cast<long>(f.G.Nr + f.G.g) * (f.G.Nz + f.G.g);
-        hipLaunchKernelGGL(k_ell_inject, dim3(blocks(n)), dim3(kBlk), 0, st, f.G, b.G, b.P.u, f.P.u, f.P.v,
+        hipLaunchKernelGGL(k_ell_inject, dim3(blocks(n)), dim3(kBlk), 0, st, f.G, b.G, u_now(b), u_now(f), v_now(f),
                            h->p.interporder);
         ELLRC(launched("injection"));
       }
@@ -1147,7 +1476,7 @@ int ell_solve_begin(oa_handle* h, int stationary_exit, EllSolver** out) {
 
 int ell_solve_run(EllSolver* s, int* steps0, int* steps1, double* gres) { return s->solve(steps0, steps1, gres); }
 
-const double* ell_solution(const EllSolver* s, int level) { return s->lev[level].P.u; }
+const double* ell_solution(const EllSolver* s, int level) { return s->u_now(s->lev[level]); }
 
 void ell_solve_end(EllSolver* s) { delete s; }
 

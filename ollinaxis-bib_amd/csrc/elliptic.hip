@@ -379,13 +379,16 @@ __global__ void __launch_bounds__(kBlk) k_ell_iter_fb(EllStepArgs a, EllCtl* ctl
 // the last one leaves the block.  Bound by latency: a level step of 128 x 256
 // took a copy of 4 us and three launches of 6 us, each mostly its start and
 // one round trip to memory.  With it the solve of a pulse on two such levels
-// went from 233 to 110 ms, a Brill wave's on five levels of 256 x 512 from 3.3
+// went from 233 to 93 ms, a Brill wave's on five levels of 256 x 512 from 3.3
 // to 2.1 s.  The states rotate through three planes instead
 // of being copied: a step reads the current one, finebound also reads the one
 // before at its own zone (time level t-1; no strips), and the result goes to
 // the third.  The level's clock rotates with them.
-constexpr int kEsTile = 16, kEsHalo = 9, kEsW = kEsTile + 2 * kEsHalo, kEsSize = kEsW * kEsW, kEsBlock = 512;
-constexpr int kEsZone = 2;         // zone points per thread, at most (540 in a block)
+// Tiles of 8 x 16 points where 16 x 16 would leave compute units without a
+// block: half as much again per point, but shorter chains and twice the blocks
+// (128 x 256 with equatorial symmetry: 128 blocks 11.0 us, 256 blocks 9.8).
+constexpr int kEsTile = 16, kEsHalo = 9, kEsW = kEsTile + 2 * kEsHalo;
+constexpr int kEsFill = 256;       // blocks that give every compute unit one
 
 struct EllStep1Args {
   KGrid G, Gc;
@@ -423,8 +426,10 @@ struct EsPlane {                     // a staged plane
   __device__ __forceinline__ double operator()(int i, int j) const { return p[(i - ei) * kEsW + (j - ej)]; }
 };
 
+template <int TI, int kEsBlock>
 __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl* ctl) {
-  if (ctl->done) return;
+  constexpr int kEsSize = (TI + 2 * kEsHalo) * kEsW;
+  constexpr int kEsZone = ((TI + 12) * (kEsTile + 12) + kEsBlock - 1) / kEsBlock;   // zone points per thread
   __shared__ double st[6][kEsSize];  // u, v: start, first and second iteration
   __shared__ double sS1[kEsSize];
   const KGrid& G = a.G;
@@ -433,10 +438,13 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
   // the last tiles end at the level's edge (and overlap the ones before, with
   // the same values): the one-sided stencils there reach 5 points inwards,
   // more than the 3 of an iteration's halo
-  const int i0 = max(min(1 + bi * kEsTile, G.Nr - kEsTile + 1), 1);
+  const int i0 = max(min(1 + bi * TI, G.Nr - TI + 1), 1);
   const int j0 = max(min(G.jlo + bj * kEsTile, G.Nz - kEsTile + 1), G.jlo);
   const int ei = i0 - kEsHalo, ej = j0 - kEsHalo;
-  if (blockIdx.x == 0 && t == 0) {                                    // :997-1004
+  // a block alone on its compute unit looks at the rule once its loads are under way
+  const int done = ctl->done;
+  if (TI == kEsTile && done) return;
+  if (blockIdx.x == 0 && t == 0) {                                    // :997-1004; not read once done
     EllClock c = *a.clk;
     c.t2 = c.t1;
     c.t1 = c.t;
@@ -461,7 +469,7 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
   const bool fine = a.cclk != nullptr;
   double tp = 0.0, ct0 = 0.0, tm1 = 0.0;
   int zr = 0, zi = 0, zl = 0, zh = 0, nz = 0;   // rows of the rho strip and of the rest; columns low, high
-  const int hi_i = min(i0 + kEsTile - 1 + 6, G.Nr), lo_i = max(i0 - 6, 1);
+  const int hi_i = min(i0 + TI - 1 + 6, G.Nr), lo_i = max(i0 - 6, 1);
   const int hi_j = min(j0 + kEsTile - 1 + 6, G.Nz), lo_j = max(j0 - 6, G.jlo);
   const int wj = hi_j - lo_j + 1;
   if (fine) {
@@ -514,6 +522,7 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
       }
     }
   }
+  if (TI < kEsTile && done) return;
   __syncthreads();
   const EsPlane U0{st[0], ei, ej}, V0{st[1], ei, ej};
 #pragma unroll
@@ -522,7 +531,7 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
     const EsPlane U{st[2 * (k - 1)], ei, ej}, V{st[2 * (k - 1) + 1], ei, ej};
     double* const ou = st[k < 3 ? 2 * k : 0];   // unused on the last iteration
     double* const ov = st[k < 3 ? 2 * k + 1 : 1];
-    const int R = 3 * (3 - k), W = kEsTile + 2 * R;
+    const int R = 3 * (3 - k), H = TI + 2 * R, W = kEsTile + 2 * R;
     const double tl = ct0 + dtw;
     const bool same = fine && tp == tl;
     const int D = same ? g + 2 : g - 1;
@@ -535,7 +544,7 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
       }
       auto set = [&](int ii, int jj) {
         const int x = ii - ei, y = jj - ej;
-        if (x < 0 || x >= kEsW || y < 0 || y >= kEsW) return;
+        if (x < 0 || x >= TI + 2 * kEsHalo || y < 0 || y >= kEsW) return;
         ou[x * kEsW + y] = nu;
         ov[x * kEsW + y] = nv;
       };
@@ -546,7 +555,7 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
         if (i <= g) set(1 - i, 1 - j);
       }
     };
-    for (int q = t; q < W * W; q += kEsBlock) {
+    for (int q = t; q < H * W; q += kEsBlock) {
       const int i = i0 - R + q / W, j = j0 - R + q % W;
       if (i < 1 || i > G.Nr || j < G.jlo || j > G.Nz) continue;
       if (fine && ell_in_zone(G, D, i, j)) continue;
@@ -559,24 +568,31 @@ __global__ void __launch_bounds__(kEsBlock, 4) k_ell_step(EllStep1Args a, EllCtl
       if (k == 3 && a.base) a.sv[kk] = sv;
     }
     if (fine && nz > 0) {
-      // finebound (finebound.f90:70-400), as ell_fb_point forms it
+      // finebound (finebound.f90:70-400), as ell_fb_point forms it: the weights
+      // of the coarse value, the start of the step and the start of the one before
+      const double t0 = ct0;
+      double cp, c0, c1 = 0.0;
+      if (tm1 == 0.0) {
+        cp = (tl - t0) / (tp - t0);
+        c0 = (tl - tp) / (t0 - tp);
+      } else {
+        cp = (tl - t0) * (tl - tm1) / ((tp - t0) * (tp - tm1));
+        c0 = (tl - tp) * (tl - tm1) / ((t0 - tp) * (t0 - tm1));
+        c1 = (tl - tp) * (tl - t0) / ((tm1 - tp) * (tm1 - t0));
+      }
 #pragma unroll
       for (int z = 0; z < kEsZone; ++z) {
         const int q = t + z * kEsBlock;
         if (q >= nz) continue;
         int i, j;
         zone_point(q, i, j);
-        if (i < i0 - R || i >= i0 + kEsTile + R || j < j0 - R || j >= j0 + kEsTile + R) continue;
+        if (i < i0 - R || i >= i0 + TI + R || j < j0 - R || j >= j0 + kEsTile + R) continue;
         if (!ell_in_zone(G, D, i, j)) continue;
-        const double t0 = ct0;
         const bool inside = ell_in_zone(G, g - 1, i, j);
         const double au = zu[z][same ? 0 : 1], av = zv[z][same ? 0 : 1];
         auto in_time = [&](double aux2, double start, double before) {
-          if (tm1 == 0.0) return (tl - t0) / (tp - t0) * aux2 + (tl - tp) / (t0 - tp) * start;
-          const double b0 = inside ? start : 0.0, b1 = before;
-          return (tl - t0) * (tl - tm1) / ((tp - t0) * (tp - tm1)) * aux2 +
-                 (tl - tp) * (tl - tm1) / ((t0 - tp) * (t0 - tm1)) * b0 +
-                 (tl - tp) * (tl - t0) / ((tm1 - tp) * (tm1 - t0)) * b1;
+          if (tm1 == 0.0) return fma(cp, aux2, c0 * start);
+          return fma(c1, before, fma(cp, aux2, c0 * (inside ? start : 0.0)));
         };
         keep(i, j, in_time(au, U0(i, j), mu[z]), in_time(av, V0(i, j), mv[z]));
       }
@@ -630,11 +646,16 @@ __global__ void __launch_bounds__(kBlk) k_ell_restrict(EllRsArgs a, const EllCtl
 // Residual and change of the base level after a coarse step, per block: sum
 // of sv^2 (i in [1, Nr-g], j in [1, Nz-g], wave_elliptic.f90:321-341), max |u
 // - up| and max |u| over the same range.  The last block to arrive combines
-// the blocks' partials in block order and applies the stopping rule.
+// the blocks' partials in a fixed order and applies the stopping rule.
 // Reference (:303): continue while step < 100 or (gres > WE_epsilon and step <
 // WE_maxiter) -- a NaN residual stops.  Stationary rule (all-levels phase
 // only, when enabled): stop once the window maximum over 100 steps of max|u -
 // up| / max|u| is at most 1e-12 and above half the previous window's.
+//
+// Bound by latency (the launch, two round trips, the arrivals at one counter
+// and the partials' way between the dies): few blocks, one point a thread up
+// to 128 x 256, reductions in registers.  256 blocks with trees in LDS and a
+// serial sum took 11.4 us of a step of 128 x 256, this 5.2.
 struct EllCheckArgs {
   KGrid G;
   const double *sv, *u, *up;
@@ -642,66 +663,64 @@ struct EllCheckArgs {
   double nntot, eps;
   int maxiter;
 };
-constexpr int kEllParts = 256;
-static_assert(kEllParts == kBlk, "one partial per thread of the last block");
+constexpr int kEllParts = 256;     // partials the SOR sweep leaves
+constexpr int kEcBlock = 512, kEcWaves = kEcBlock / 64, kEcBlocks = 128;
 
-__global__ void __launch_bounds__(kBlk) k_ell_check(EllCheckArgs a, EllCtl* ctl) {
+struct EllNorms {
+  double sq, du, mu;
+  __device__ __forceinline__ void add(const EllNorms& o) {
+    sq += o.sq;
+    du = fmax(du, o.du);
+    mu = fmax(mu, o.mu);
+  }
+  template <int N>
+  __device__ __forceinline__ void fold() {   // over the first N lanes, in a fixed order
+#pragma unroll
+    for (int m = N / 2; m > 0; m >>= 1) add(EllNorms{__shfl_xor(sq, m), __shfl_xor(du, m), __shfl_xor(mu, m)});
+  }
+};
+
+__global__ void __launch_bounds__(kEcBlock) k_ell_check(EllCheckArgs a, EllCtl* ctl) {
   if (ctl->done) return;
-  __shared__ double ssq[kBlk], sdu[kBlk], smu[kBlk];
-  __shared__ unsigned last;
+  __shared__ EllNorms wave[kEcWaves];
   const KGrid& G = a.G;
-  const int ni = G.Nr - G.g, nj = G.Nz - G.g;
-  const long n = static_cast<long>(ni) * nj;
-  double sq = 0.0, du = 0.0, mu = 0.0;
-  for (long q = static_cast<long>(blockIdx.x) * kBlk + threadIdx.x; q < n; q += static_cast<long>(gridDim.x) * kBlk) {
-    const int i = 1 + static_cast<int>(q / nj), j = 1 + static_cast<int>(q % nj);
-    const long k = IDX(G, i, j);
-    const double s = a.sv[k];
-    sq += s * s;
-    du = fmax(du, fabs(a.u[k] - a.up[k]));
-    mu = fmax(mu, fabs(a.u[k]));
+  const int ni = G.Nr - G.g, nj = G.Nz - G.g, n = ni * nj, t = static_cast<int>(threadIdx.x);
+  EllNorms m{0.0, 0.0, 0.0};
+  for (int q = static_cast<int>(blockIdx.x) * kEcBlock + t; q < n; q += static_cast<int>(gridDim.x) * kEcBlock) {
+    const long k = IDX(G, 1 + q / nj, 1 + q % nj);
+    const double s = a.sv[k], u = a.u[k];
+    m.add(EllNorms{s * s, fabs(u - a.up[k]), fabs(u)});
   }
-  const int t = static_cast<int>(threadIdx.x);
-  auto tree = [&](bool sum) {
-    for (int h = kBlk / 2; h > 0; h >>= 1) {
-      if (t < h) {
-        if (sum) ssq[t] += ssq[t + h];
-        sdu[t] = fmax(sdu[t], sdu[t + h]);
-        smu[t] = fmax(smu[t], smu[t + h]);
-      }
-      __syncthreads();
-    }
-  };
-  ssq[t] = sq; sdu[t] = du; smu[t] = mu;
+  m.fold<64>();
+  if ((t & 63) == 0) wave[t >> 6] = m;
   __syncthreads();
-  tree(true);
+  if (t >= 64) return;
+  m = wave[t & (kEcWaves - 1)];
+  m.fold<kEcWaves>();
+  unsigned arrived = 0;
   if (t == 0) {
-    a.part[3 * blockIdx.x] = ssq[0];
-    a.part[3 * blockIdx.x + 1] = sdu[0];
-    a.part[3 * blockIdx.x + 2] = smu[0];
+    double* part = a.part + 3 * blockIdx.x;
+    part[0] = m.sq;
+    part[1] = m.du;
+    part[2] = m.mu;
     __threadfence();
-    last = atomicAdd(&ctl->arrived, 1u);
+    arrived = atomicAdd(&ctl->arrived, 1u);
   }
-  __syncthreads();
-  if (last != gridDim.x - 1) return;
+  if (__builtin_amdgcn_readfirstlane(arrived) != gridDim.x - 1) return;
   __threadfence();
-  ssq[t] = a.part[3 * t];
-  sdu[t] = a.part[3 * t + 1];
-  smu[t] = a.part[3 * t + 2];
-  __syncthreads();
-  tree(false);
+  m = EllNorms{0.0, 0.0, 0.0};
+  for (int b = t; b < static_cast<int>(gridDim.x); b += 64)
+    m.add(EllNorms{a.part[3 * b], a.part[3 * b + 1], a.part[3 * b + 2]});
+  m.fold<64>();
   if (t != 0) return;
-  double total = 0.0;
-#pragma unroll 16
-  for (int b = 0; b < kEllParts; ++b) total += ssq[b];
   EllCtl& c = *ctl;
   c.arrived = 0u;
   const int step = c.step + 1;
-  const double gres = sqrt(total / a.nntot);
+  const double gres = sqrt(m.sq / a.nntot);
   const bool more = (step < 100) || (gres > a.eps && step < a.maxiter);
   int done = more ? 0 : 1;
   if (!done && c.stationary) {
-    const double rel = sdu[0] / smu[0];
+    const double rel = m.du / m.mu;
     if (rel > c.wmax) c.wmax = rel;
     if (step % 100 == 0) {
       if (c.wmax <= 1.0e-12 && c.wmax > 0.5 * c.wprev) done = 1;
@@ -1089,8 +1108,9 @@ struct EllSolver {
       s.tab[1] = h->L[level].fbtab[1];
       s.cclk = c.clk + c.cur;
     }
-    const int nbi = (a.G.Nr + kEsTile - 1) / kEsTile;
-    hipLaunchKernelGGL(k_ell_step, dim3(nbi * s.nbj), dim3(kEsBlock), 0, st, s, ctl);
+    const int nb16 = (a.G.Nr + 15) / 16 * s.nbj, nb8 = (a.G.Nr + 7) / 8 * s.nbj;
+    if (nb16 < kEsFill) hipLaunchKernelGGL((k_ell_step<8, 512>), dim3(nb8), dim3(512), 0, st, s, ctl);
+    else hipLaunchKernelGGL((k_ell_step<16, 512>), dim3(nb16), dim3(512), 0, st, s, ctl);
     ELLRC(launched("ICN step"));
     a.cur = nxt;
     return OA_OK;
@@ -1221,7 +1241,9 @@ struct EllSolver {
     c.nntot = static_cast<double>(b.G.Nr) * static_cast<double>(b.G.Nz);
     c.eps = h->p.WE_epsilon;
     c.maxiter = h->p.WE_maxiter;
-    hipLaunchKernelGGL(k_ell_check, dim3(nparts), dim3(kBlk), 0, st, c, ctl);
+    const long n = static_cast<long>(b.G.Nr - b.G.g) * (b.G.Nz - b.G.g);
+    const int nb = static_cast<int>(std::min<long>((n + kEcBlock - 1) / kEcBlock, kEcBlocks));
+    hipLaunchKernelGGL(k_ell_check, dim3(nb), dim3(kEcBlock), 0, st, c, ctl);
     return launched("residual and stopping rule");
   }
 

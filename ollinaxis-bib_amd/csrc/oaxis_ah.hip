@@ -28,10 +28,11 @@
 //     needs a shot it has not got, it launches the whole speculative
 //     continuation at once: during the march, the next positions down the
 //     axis; during the bisection, the full tree of the next bisection steps,
-//     as deep as keeps every search's tree resident on the device at once
-//     (kAhResident waves in all, at most kAhMaxDepth steps).  The walk then takes exactly the reference's path
-//     through those results, so the sequence of shots and every decision
-//     are the reference's; unused shots are discarded.
+//     as deep as gives every shot of every search a SIMD of its own
+//     (kAhResident waves in all, at most kAhMaxDepth steps).  The walk then
+//     takes exactly the reference's path through those results, so the
+//     sequence of shots and every decision are the reference's; shots that
+//     finished ones exclude end early, and unused ones are discarded.
 //
 // Floating-point contraction is off in this file, so the sources and the
 // interpolation round like the oracle's IEEE build of the same expressions.
@@ -64,7 +65,11 @@ constexpr int kAhNthetaMax = 50000;                 // Nthetamax (:350)
 constexpr int kAhMaxSteps = 4 * kAhNthetaMax;
 constexpr int kAhScanChunk = 1024;                  // march positions per launch
 constexpr int kAhMaxDepth = 11;                     // bisection steps per launch, at most
-constexpr int kAhResident = 2048;                   // shot waves resident at once (256 CUs x 8)
+// Shots of one launch: one wave to a SIMD (256 CUs x 4).  A shot is bound by
+// the issue of its own serial chain, so two waves on a SIMD take twice as long
+// (a tree of 11 steps 12.0 ms where one shot alone took 6.0), for one
+// bisection step more.
+constexpr int kAhResident = 1024;
 constexpr int kShotBlock = 64;
 
 // interpolated quantities, in ah_source's order
@@ -92,12 +97,78 @@ struct ShotIn {
   double zinit, zcenter;
   double* theta;                      // when not null: accepted points (kAhNthetaMax + 1)
   double* rad;
+  // the shot's place in its search's speculation: number at of n shots, the
+  // first of which is the launch's shot base
+  int kind, base, at, n;
+  double drada;                       // kShotTree: the sign the bisection compares with
 };
+enum ShotKind { kShotAlone = 0, kShotMarch, kShotTree };
 
 struct ShotOut {
   double dradlast, area;
   int err, ntheta;
 };
+constexpr int kShotDropped = -1;      // ShotOut::err: not integrated to its end
+
+// Speculative shots that can no longer be asked for end early (two levels of
+// 128 x 256: the march's launch 21.5 -> 18.1 ms, the first tree's 25.9 -> 18.4
+// together with its smaller depth).  A march ends
+// at the first pair of neighbours whose end slopes differ in sign, so the
+// shots past a finished such pair are dropped; a node of the bisection's tree
+// sends the walk into one of its two subtrees, so a finished node drops the
+// other.  Only shots whose need is excluded by finished ones are dropped, and
+// the first shot of a launch never is, so each launch brings the walk on; a
+// dropped shot that is asked for later all the same is launched again.  Each
+// shot looks once per step, with a load that the step's sources hide; nothing
+// waits.  done: one word per shot (kShotMarch: 1 once its result is out;
+// kShotTree: 1 and 2 drop the left and the right subtree), and after those of
+// the launch's `total` shots one per shot again, of which a march uses that of
+// its first shot: how many of its shots are from the nearest end on.
+
+__device__ __forceinline__ int shot_word(const int* done, int q) {
+  return __hip_atomic_load(done + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// each lane looks at one word: lane 0 at the march's, lane l at the tree's
+// ancestor l + 1 steps up
+__device__ __forceinline__ int shot_look(const ShotIn& s, const int* done, int total) {
+  const int lane = static_cast<int>(threadIdx.x);
+  if (s.kind == kShotMarch) return lane == 0 ? shot_word(done, total + s.base) : 0;
+  if (s.kind != kShotTree || lane >= kAhMaxDepth) return 0;
+  const int up = (s.at + 1) >> (lane + 1);
+  return up > 0 ? shot_word(done, s.base + up - 1) : 0;
+}
+
+__device__ __forceinline__ bool shot_dropped(const ShotIn& s, int word) {
+  const int lane = static_cast<int>(threadIdx.x);
+  bool drop = false;
+  if (s.kind == kShotMarch) {
+    drop = lane == 0 && word > 0 && s.at > s.n - word;
+  } else if (s.kind == kShotTree) {
+    const bool right = (((s.at + 1) >> lane) & 1) != 0;    // the child of that ancestor the shot is below
+    drop = lane < kAhMaxDepth && (word & (right ? 2 : 1)) != 0;
+  }
+  return __any(drop);
+}
+
+// a finished shot's result d, by one lane; out holds it already
+__device__ __forceinline__ void shot_publish(const ShotIn& s, int* done, int total, const ShotOut* out, double d) {
+  if (s.kind == kShotTree) {
+    const double p = s.drada * d;
+    if (p <= 0.0) atomicOr(done + s.base + s.at, 2);
+    else if (p > 0.0) atomicOr(done + s.base + s.at, 1);
+  } else if (s.kind == kShotMarch) {
+    __threadfence();
+    atomicOr(done + s.base + s.at, 1);
+    for (int q = s.at - 1; q <= s.at + 1; q += 2) {
+      if (q < 0 || q >= s.n || !(shot_word(done, s.base + q) & 1)) continue;
+      __threadfence();
+      const double o = __hip_atomic_load(&out[s.base + q].dradlast, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int end = s.at > q ? s.at : q;
+      if (!(d * o >= 0.0)) atomicMax(done + total + s.base, s.n - end);
+    }
+  }
+}
 
 // ------------------------------------------------------------ derived planes
 // psi = exp(phi) (auxiliary_geometry.f90:236-242), Dr/Dz of phi (:176-231),
@@ -202,6 +273,34 @@ struct AhCell {
 // near the level's edges (or with interporder = bilinear), else bicubic
 // Lagrange weights.  Formed once per point; ah_combine applies it to the
 // records of one quantity with the reference's expressions.
+//
+// Quotients by one divisor share its reciprocal: two Newton steps on the
+// hardware's estimate, then per quotient a product and one residual correction
+// (Markstein 1990), which rounds correctly wherever numerator, divisor and
+// quotient are normal numbers; three instructions instead of eleven.  A
+// division by zero or of an infinity gives NaN, which the sources refuse as
+// they refuse an infinity.
+struct AhRecip {
+  double d, y;
+  __device__ __forceinline__ explicit AhRecip(double div) : d(div) {
+    y = __builtin_amdgcn_rcp(d);
+    y = fma(y, fma(-d, y, 1.0), y);
+    y = fma(y, fma(-d, y, 1.0), y);
+  }
+  __device__ __forceinline__ AhRecip(double div, double recip) : d(div), y(recip) {}
+  __device__ __forceinline__ double of(double x) const {
+    const double q = x * y;
+    return fma(fma(-d, q, x), y, q);
+  }
+};
+
+// x / n for the bicubic weights' n, 1 <= |n| <= 3
+__device__ __forceinline__ double ah_over(double x, int n) {
+  const int m = n < 0 ? -n : n;
+  const double q = (m == 3) ? AhRecip(3.0, 1.0 / 3.0).of(x) : (m == 2) ? 0.5 * x : x;
+  return n < 0 ? -q : q;
+}
+
 struct AhPlan {
   int lev, i0, j0, mode;              // mode 0: node copy, 1: bilinear, 2: bicubic
   double auxr, auxz;
@@ -213,9 +312,10 @@ __device__ __forceinline__ void ah_plan(const AhLevel& L, int order, double r0, 
   const int g = G.g;
   const double r1g = (static_cast<double>(1 - g) - 0.5) * G.dr;
   const double z1g = (static_cast<double>(1 - g) - G.zoff) * G.dz;
-  const int i0 = static_cast<int>((r0 - r1g) / G.dr) + 1 - g;
+  const AhRecip dr(G.dr), dz(G.dz);
+  const int i0 = static_cast<int>(dr.of(r0 - r1g)) + 1 - g;
   const double deltar = r0 - (static_cast<double>(i0) - 0.5) * G.dr;
-  const int j0 = static_cast<int>((z0 - z1g) / G.dz) + 1 - g;
+  const int j0 = static_cast<int>(dz.of(z0 - z1g)) + 1 - g;
   const double deltaz = z0 - (static_cast<double>(j0) - G.zoff) * G.dz;
   P.i0 = i0;
   P.j0 = j0;
@@ -227,7 +327,7 @@ __device__ __forceinline__ void ah_plan(const AhLevel& L, int order, double r0, 
   }
   const bool lin = ((L.rmax - r0) < G.dr) || ((L.zmax - z0) < G.dz) || ((r0 - L.rmin) < G.dr) ||
                    ((z0 - L.zmin) < G.dz);
-  const double auxr = deltar / G.dr, auxz = deltaz / G.dz;
+  const double auxr = dr.of(deltar), auxz = dz.of(deltaz);
   P.auxr = auxr;
   P.auxz = auxz;
   if (order == OA_INTERP_BILINEAR || lin) {
@@ -241,7 +341,7 @@ __device__ __forceinline__ void ah_plan(const AhLevel& L, int order, double r0, 
 #pragma unroll
     for (int m = -1; m <= 2; ++m) {
       if (m == i) continue;
-      wr = wr * (auxr - static_cast<double>(m)) / static_cast<double>(i - m);
+      wr = ah_over(wr * (auxr - static_cast<double>(m)), i - m);
     }
 #pragma unroll
     for (int j = -1; j <= 2; ++j) {
@@ -249,7 +349,7 @@ __device__ __forceinline__ void ah_plan(const AhLevel& L, int order, double r0, 
 #pragma unroll
       for (int n = -1; n <= 2; ++n) {
         if (n == j) continue;
-        aux = aux * (auxz - static_cast<double>(n)) / static_cast<double>(j - n);
+        aux = ah_over(aux * (auxz - static_cast<double>(n)), j - n);
       }
       P.w[i + 1][j + 1] = aux;
     }
@@ -364,8 +464,10 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
   const double smallpi = M_PI;
 
   const double interp_psi4 = (v[AF_psi] * v[AF_psi]) * (v[AF_psi] * v[AF_psi]);
+  const double rc2 = rc * rc, zc2 = zc * zc, rad2 = rad * rad;
+  const AhRecip o_rad(rad), o_rad2(rad2), o_psi4(interp_psi4);
   double Dphi[3];                                                                // :2247-2249
-  Dphi[0] = (rc * v[AF_Drphi] + zc * v[AF_Dzphi]) / rad;
+  Dphi[0] = o_rad.of(rc * v[AF_Drphi] + zc * v[AF_Dzphi]);
   Dphi[1] = (zc * v[AF_Drphi] - rc * v[AF_Dzphi]);
   Dphi[2] = zero;
 
@@ -373,12 +475,11 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
   const double iB = v[AF_B], iDrB = v[AF_DrB], iDzB = v[AF_DzB];
   const double iC = v[AF_C], iDrC = v[AF_DrC], iDzC = v[AF_DzC];
   const double iH = v[AF_H], iDrH = v[AF_DrH], iDzH = v[AF_DzH];
-  const double rc2 = rc * rc, zc2 = zc * zc, rad2 = rad * rad;
 
   double gd[3][3], gu[3][3];                                                     // :2320-2340
-  gd[0][0] = (rc2 * iA + zc2 * iB + two * rc2 * zc * iC) / rad2;
+  gd[0][0] = o_rad2.of(rc2 * iA + zc2 * iB + two * rc2 * zc * iC);
   gd[1][1] = (zc2 * iA + rc2 * iB - two * rc2 * zc * iC);
-  gd[0][1] = rc * (zc * (iA - iB) + (zc2 - rc2) * iC) / rad;
+  gd[0][1] = o_rad.of(rc * (zc * (iA - iB) + (zc2 - rc2) * iC));
   gd[2][2] = rc2 * iH;
   gd[0][2] = zero;
   gd[1][2] = zero;
@@ -387,10 +488,11 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
   gd[2][1] = gd[1][2];
   if (th != zero && th != smallpi) {                                             // :2345-2378
     const double aux = gd[0][0] * gd[1][1] - gd[0][1] * gd[0][1];
-    gu[0][0] = gd[1][1] / aux;
-    gu[1][1] = gd[0][0] / aux;
+    const AhRecip o_aux(aux);
+    gu[0][0] = o_aux.of(gd[1][1]);
+    gu[1][1] = o_aux.of(gd[0][0]);
     gu[2][2] = one / gd[2][2];
-    gu[0][1] = -gd[0][1] / aux;
+    gu[0][1] = o_aux.of(-gd[0][1]);
   } else {
     gu[0][0] = one / gd[0][0];
     gu[1][1] = one / gd[1][1];
@@ -405,26 +507,26 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
 
   double Dg[3][3][3];                                                            // :2388-2472
   double diffr, diffz;
-  diffr = (two * rc * iA + rc2 * iDrA + zc2 * iDrB + two * rc * zc * (two * iC + rc * iDrC) - two * rc * gd[0][0]) / rad2;
-  diffz = (rc2 * iDzA + two * zc * iB + zc2 * iDzB + two * rc2 * (iC + zc * iDzC) - two * zc * gd[0][0]) / rad2;
-  Dg[0][0][0] = (rc * diffr + zc * diffz) / rad;
+  diffr = o_rad2.of(two * rc * iA + rc2 * iDrA + zc2 * iDrB + two * rc * zc * (two * iC + rc * iDrC) - two * rc * gd[0][0]);
+  diffz = o_rad2.of(rc2 * iDzA + two * zc * iB + zc2 * iDzB + two * rc2 * (iC + zc * iDzC) - two * zc * gd[0][0]);
+  Dg[0][0][0] = o_rad.of(rc * diffr + zc * diffz);
   Dg[1][0][0] = (zc * diffr - rc * diffz);
   diffr = (two * rc * iB + rc2 * iDrB + zc2 * iDrA - two * rc * zc * (two * iC + rc * iDrC));
   diffz = (rc2 * iDzB + two * zc * iA + zc2 * iDzA - two * rc2 * (iC + zc * iDzC));
-  Dg[0][1][1] = (rc * diffr + zc * diffz) / rad;
+  Dg[0][1][1] = o_rad.of(rc * diffr + zc * diffz);
   Dg[1][1][1] = (zc * diffr - rc * diffz);
   {
-    const double q = rc / rad;
-    diffr = ((one - q * q) * (zc * (iA - iB) + (zc2 - rc2) * iC) +
-             rc * (zc * (iDrA - iDrB) + (zc2 - rc2) * iDrC - two * rc * iC)) / rad;
-    diffz = q * (-(zc / rad2) * (zc * (iA - iB) + (zc2 - rc2) * iC) + (iA - iB) + zc * (iDzA - iDzB) +
+    const double q = o_rad.of(rc);
+    diffr = o_rad.of((one - q * q) * (zc * (iA - iB) + (zc2 - rc2) * iC) +
+                     rc * (zc * (iDrA - iDrB) + (zc2 - rc2) * iDrC - two * rc * iC));
+    diffz = q * (-o_rad2.of(zc) * (zc * (iA - iB) + (zc2 - rc2) * iC) + (iA - iB) + zc * (iDzA - iDzB) +
                  (zc2 - rc2) * iDzC + two * zc * iC);
   }
-  Dg[0][0][1] = (rc * diffr + zc * diffz) / rad;
+  Dg[0][0][1] = o_rad.of(rc * diffr + zc * diffz);
   Dg[1][0][1] = (zc * diffr - rc * diffz);
   diffr = rc * (two * iH + rc * iDrH);
   diffz = rc2 * iDzH;
-  Dg[0][2][2] = (rc * diffr + zc * diffz) / rad;
+  Dg[0][2][2] = o_rad.of(rc * diffr + zc * diffz);
   Dg[1][2][2] = (zc * diffr - rc * diffz);
 #pragma unroll
   for (int d = 0; d < 2; ++d) {
@@ -440,9 +542,9 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
     for (int j = 0; j < 3; ++j) Dg[2][i][j] = zero;
 
   double Kd[3][3];                                                               // :2510-2530
-  Kd[0][0] = (rc2 * v[AF_KA] + zc2 * v[AF_KB] + two * rc2 * zc * v[AF_KC]) / rad2;
+  Kd[0][0] = o_rad2.of(rc2 * v[AF_KA] + zc2 * v[AF_KB] + two * rc2 * zc * v[AF_KC]);
   Kd[1][1] = (zc2 * v[AF_KA] + rc2 * v[AF_KB] - two * rc2 * zc * v[AF_KC]);
-  Kd[0][1] = rc * (zc * (v[AF_KA] - v[AF_KB]) + (zc2 - rc2) * v[AF_KC]) / rad;
+  Kd[0][1] = o_rad.of(rc * (zc * (v[AF_KA] - v[AF_KB]) + (zc2 - rc2) * v[AF_KC]));
   Kd[2][2] = rc2 * v[AF_KH];
   Kd[0][2] = zero;
   Kd[1][2] = zero;
@@ -452,8 +554,8 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
 
   double DF[3];                                                                  // :2537-2552
 #pragma unroll
-  for (int i = 0; i < 3; ++i) DF[i] = (gu[0][i] - gu[1][i] * dh) / interp_psi4;
-  const double u2 = (gu[0][0] - two * gu[0][1] * dh + gu[1][1] * dh * dh) / interp_psi4;
+  for (int i = 0; i < 3; ++i) DF[i] = o_psi4.of(gu[0][i] - gu[1][i] * dh);
+  const double u2 = o_psi4.of(gu[0][0] - two * gu[0][1] * dh + gu[1][1] * dh * dh);
   const double u = std::sqrt(std::fabs(u2));
   const double denom = (gu[0][0] * gu[1][1] - gu[0][1] * gu[0][1]) / (interp_psi4 * interp_psi4);
 
@@ -482,7 +584,7 @@ __device__ int ah_source_math(double rad, double dh, double th, double rc, doubl
 #pragma unroll
   for (int q = 0; q < 5; ++q) {
     const int i = kIJ[q][0], j = kIJ[q][1];
-    s = s + u2 * gu[i][j] * (Gam[0][i][j] - Gam[1][i][j] * dh) / interp_psi4;
+    s = s + o_psi4.of(u2 * gu[i][j] * (Gam[0][i][j] - Gam[1][i][j] * dh));
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -529,8 +631,11 @@ __device__ int ah_source(const AhCtx& c, double rad, double dh, double th, doubl
 // zinit.  The reference's "local extrapolation" (:672-677) writes the slot
 // after the accepted one, which the next step overwrites before reading, so
 // it has no effect and is not restated.
-__device__ ShotOut ah_integrate(const AhCtx& c, double zinit, double zcenter, double* th_out, double* rad_out,
-                                double* sv, double* xs, int* xe) {
+__device__ ShotOut ah_integrate(const ShotIn& in, const int* done, int total, double* sv, double* xs, int* xe) {
+  const AhCtx& c = *in.ctx;
+  const double zinit = in.zinit, zcenter = in.zcenter;
+  double* const th_out = in.theta;
+  double* const rad_out = in.rad;
   const double zero = 0.0, half = 0.5, two = 2.0;
   const double smallpi = M_PI;
   double rad = std::fabs(zinit - zcenter);
@@ -564,82 +669,86 @@ __device__ ShotOut ah_integrate(const AhCtx& c, double zinit, double zcenter, do
       err = 1;
       break;
     }
+    const int word = shot_look(in, done, total);
     if (zcenter >= zero) {
       if (theta + dth > thetafinal) dth = thetafinal - theta;
     } else {
       if (theta + dth < thetafinal) dth = thetafinal - theta;
     }
     const double dth2 = half * dth;
-    double rad1, drad1, area1, drad_aux;
-    double k_1, k_2, k_3, k_4, l_1, l_2, l_3, l_4, m_1, m_2, m_3, m_4;
-    if ((err = ah_source(c, rad, drad, theta, zcenter, sdh, sarea, sv, cell))) break;
-    k_1 = dth * drad;
-    l_1 = dth * sdh;
-    m_1 = std::fabs(dth2) * sarea;
-    // The large step's last three stages and the first small step's last
-    // three are independent: the upper half-wave runs the large step, the
-    // lower half the small one, in one instruction stream (step h, first
-    // stage k1/l1 per half, in the reference's expressions).  An error in
-    // either ends the step as the reference's first error would: nothing of
+    // Eight sequential source evaluations: the first stage of both step sizes,
+    // then their last three side by side (they are independent: the upper
+    // half-wave runs the large step, the lower half the first small one, step
+    // h), then the four stages of the second small step on every lane.  One
+    // loop over the stages, so that the sources are in the code once: eight
+    // copies were 94 KB, more than the instruction cache holds (with the shared
+    // reciprocals, one shot 6.0 -> 4.9 ms).  An error in
+    // any stage ends the step as the reference's first error would: nothing of
     // the step is kept.
-    {
-      const bool big = (threadIdx.x >> 5) != 0;
-      const double h = big ? dth : dth2;
-      const double k1 = big ? k_1 : half * k_1;
-      const double l1 = big ? l_1 : half * l_1;
-      int e = ah_source(c, rad + 0.5 * k1, drad + 0.5 * l1, theta + 0.5 * h, zcenter, sdh, sarea, sv, cell);
-      k_2 = h * (drad + 0.5 * l1);
-      l_2 = h * sdh;
-      m_2 = std::fabs(dth2) * sarea;
-      e |= ah_source(c, rad + 0.5 * k_2, drad + 0.5 * l_2, theta + 0.5 * h, zcenter, sdh, sarea, sv, cell);
-      k_3 = h * (drad + 0.5 * l_2);
-      l_3 = h * sdh;
-      m_3 = std::fabs(dth2) * sarea;
-      e |= ah_source(c, rad + k_3, drad + l_3, theta + h, zcenter, sdh, sarea, sv, cell);
-      k_4 = h * (drad + l_3);
-      l_4 = h * sdh;
-      m_4 = std::fabs(dth2) * sarea;
-      // exchange: the small step's (rad1, drad1, area1), the large step's
-      // drad_aux and both error flags reach every lane
-      if (threadIdx.x == 0) {
-        xs[0] = rad + sixth * (k1 + 2.0 * k_2 + 2.0 * k_3 + k_4);
-        xs[1] = drad + sixth * (l1 + 2.0 * l_2 + 2.0 * l_3 + l_4);
-        xs[2] = area + sixth * (m_1 + 2.0 * m_2 + 2.0 * m_3 + m_4);
-        xe[0] = e;
+    const bool big = (threadIdx.x >> 5) != 0;
+    double h = dth, rad0 = rad, drad0 = drad, area0 = area, drad_aux = 0.0;
+    double k = 0.0, l = 0.0, sk = 0.0, sl = 0.0, sm = 0.0;    // this stage's increments and the weighted sums
+    int e = 0;
+#pragma clang loop unroll(disable)
+    for (int stage = 0; stage < 8; ++stage) {
+      const int sub = stage & 3;
+      const double c1 = (sub == 0) ? 0.0 : (sub == 3) ? 1.0 : 0.5;
+      const double at = (stage < 4) ? c1 * h : (sub == 0 || sub == 3) ? dth : 1.5 * dth2;
+      const double d = drad0 + c1 * l;
+      e |= ah_source(c, rad0 + c1 * k, d, theta + at, zcenter, sdh, sarea, sv, cell);
+      if (e && (stage == 0 || stage > 3)) break;
+      k = h * d;
+      l = h * sdh;
+      const double m = std::fabs(dth2) * sarea;
+      if (sub == 0) {
+        if (stage == 0 && !big) {
+          h = dth2;
+          k = half * k;
+          l = half * l;
+        }
+        sk = k;
+        sl = l;
+        sm = m;
+      } else {
+        const double w = (sub == 3) ? 1.0 : 2.0;
+        sk = sk + w * k;
+        sl = sl + w * l;
+        sm = sm + w * m;
       }
-      if (threadIdx.x == 32) {
-        xs[3] = drad + sixth * (l1 + 2.0 * l_2 + 2.0 * l_3 + l_4);
-        xe[1] = e;
+      if (stage == 3) {
+        // exchange: the small step's end, the large step's drad_aux and both
+        // error flags reach every lane
+        if (threadIdx.x == 0) {
+          xs[0] = rad + sixth * sk;
+          xs[1] = drad + sixth * sl;
+          xs[2] = area + sixth * sm;
+          xe[0] = e;
+        }
+        if (threadIdx.x == 32) {
+          xs[3] = drad + sixth * sl;
+          xe[1] = e;
+        }
+        __syncthreads();
+        e = xe[0] | xe[1];
+        rad0 = xs[0];
+        drad0 = xs[1];
+        area0 = xs[2];
+        drad_aux = xs[3];
+        __syncthreads();
+        if (e) break;
+        h = dth2;
+        k = 0.0;
+        l = 0.0;
       }
-      __syncthreads();
-      err = xe[0] | xe[1];
-      rad1 = xs[0];
-      drad1 = xs[1];
-      area1 = xs[2];
-      drad_aux = xs[3];
-      __syncthreads();
     }
-    if (err) break;
-
-    if ((err = ah_source(c, rad1, drad1, theta + dth, zcenter, sdh, sarea, sv, cell))) break;
-    k_1 = dth2 * drad1;
-    l_1 = dth2 * sdh;
-    m_1 = std::fabs(dth2) * sarea;
-    if ((err = ah_source(c, rad1 + 0.5 * k_1, drad1 + 0.5 * l_1, theta + 1.5 * dth2, zcenter, sdh, sarea, sv, cell))) break;
-    k_2 = dth2 * (drad1 + 0.5 * l_1);
-    l_2 = dth2 * sdh;
-    m_2 = std::fabs(dth2) * sarea;
-    if ((err = ah_source(c, rad1 + 0.5 * k_2, drad1 + 0.5 * l_2, theta + 1.5 * dth2, zcenter, sdh, sarea, sv, cell))) break;
-    k_3 = dth2 * (drad1 + 0.5 * l_2);
-    l_3 = dth2 * sdh;
-    m_3 = std::fabs(dth2) * sarea;
-    if ((err = ah_source(c, rad1 + k_3, drad1 + l_3, theta + dth, zcenter, sdh, sarea, sv, cell))) break;
-    k_4 = dth2 * (drad1 + l_3);
-    l_4 = dth2 * sdh;
-    m_4 = std::fabs(dth2) * sarea;
-    const double rad2 = rad1 + sixth * (k_1 + 2.0 * k_2 + 2.0 * k_3 + k_4);
-    const double drad2 = drad1 + sixth * (l_1 + 2.0 * l_2 + 2.0 * l_3 + l_4);
-    const double area2 = area1 + sixth * (m_1 + 2.0 * m_2 + 2.0 * m_3 + m_4);
+    if (shot_dropped(in, word)) {
+      err = kShotDropped;
+      break;
+    }
+    if ((err = e)) break;
+    const double rad2 = rad0 + sixth * sk;
+    const double drad2 = drad0 + sixth * sl;
+    const double area2 = area0 + sixth * sm;
 
     const double drad_error = std::fabs(drad2 - drad_aux);                       // :652-700
     const double eps = 1.0e-4 * (std::fabs(drad2) + std::fabs(drad_aux));
@@ -675,7 +784,7 @@ __device__ ShotOut ah_integrate(const AhCtx& c, double zinit, double zcenter, do
 // the independent stages of a step side by side (8 sequential source
 // evaluations per step instead of 11); elsewhere every lane runs the same
 // integration on the same values.
-__global__ void __launch_bounds__(kShotBlock) k_ah_shoot(const ShotIn* __restrict__ in, ShotOut* __restrict__ out,
+__global__ void __launch_bounds__(kShotBlock) k_ah_shoot(const ShotIn* __restrict__ in, ShotOut* out, int* done,
                                                          int n) {
   __shared__ double sv[2 * AF_N];
   __shared__ double xs[4];
@@ -683,8 +792,11 @@ __global__ void __launch_bounds__(kShotBlock) k_ah_shoot(const ShotIn* __restric
   const int t = static_cast<int>(blockIdx.x);
   if (t >= n) return;
   const ShotIn s = in[t];
-  const ShotOut o = ah_integrate(*s.ctx, s.zinit, s.zcenter, s.theta, s.rad, sv, xs, xe);
-  if (threadIdx.x == 0) out[t] = o;
+  const ShotOut o = ah_integrate(s, done, n, sv, xs, xe);
+  if (threadIdx.x == 0) {
+    out[t] = o;
+    if (o.err != kShotDropped) shot_publish(s, done, n, out, o.dradlast);
+  }
 }
 
 // Dz_phi at one point of one level (the moving-centre walk of
@@ -980,6 +1092,7 @@ struct AhState {
   ShotOut* h_out = nullptr;               // pinned
   ShotIn* d_in = nullptr;
   ShotOut* d_out = nullptr;
+  int* d_done = nullptr;                  // two words per shot: what its result excludes
   int cap = 0;
   double* d_theta[3] = {nullptr, nullptr, nullptr};   // last integration of horizon k
   double* d_rad[3] = {nullptr, nullptr, nullptr};
@@ -1035,6 +1148,8 @@ int ensure_capacity(AhState& a, int n) {
   if (a.h_out) (void)hipHostFree(a.h_out);
   if (a.d_in) (void)hipFree(a.d_in);
   if (a.d_out) (void)hipFree(a.d_out);
+  if (a.d_done) (void)hipFree(a.d_done);
+  a.d_done = nullptr;
   a.h_in = nullptr;
   a.h_out = nullptr;
   a.d_in = nullptr;
@@ -1044,6 +1159,7 @@ int ensure_capacity(AhState& a, int n) {
   AH_HIP(hipHostMalloc(reinterpret_cast<void**>(&a.h_out), sizeof(ShotOut) * cap, hipHostMallocDefault));
   AH_HIP(hipMalloc(reinterpret_cast<void**>(&a.d_in), sizeof(ShotIn) * cap));
   AH_HIP(hipMalloc(reinterpret_cast<void**>(&a.d_out), sizeof(ShotOut) * cap));
+  AH_HIP(hipMalloc(reinterpret_cast<void**>(&a.d_done), 2 * sizeof(int) * cap));
   a.cap = cap;
   return OA_OK;
 }
@@ -1056,7 +1172,8 @@ int run_shots(hipStream_t st, AhState& buf, const std::vector<ShotIn>& in, std::
   AH_RC(ensure_capacity(buf, n));
   std::memcpy(buf.h_in, in.data(), sizeof(ShotIn) * n);
   AH_HIP(hipMemcpyAsync(buf.d_in, buf.h_in, sizeof(ShotIn) * n, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_ah_shoot, dim3(n), dim3(kShotBlock), 0, st, buf.d_in, buf.d_out, n);
+  AH_HIP(hipMemsetAsync(buf.d_done, 0, 2 * sizeof(int) * n, st));
+  hipLaunchKernelGGL(k_ah_shoot, dim3(n), dim3(kShotBlock), 0, st, buf.d_in, buf.d_out, buf.d_done, n);
   AH_HIP(hipGetLastError());
   AH_HIP(hipMemcpyAsync(buf.h_out, buf.d_out, sizeof(ShotOut) * n, hipMemcpyDeviceToHost, st));
   AH_HIP(hipStreamSynchronize(st));
@@ -1075,6 +1192,9 @@ struct Search {
   int found = 0, errorflag = 0, shots = 0;
   double zinit = 0.0, dradlast = 0.0, last_zinit = 0.0;
   ShotRes last{0.0, 0.0, 0, 0};
+  // what the shots wanted next speculate on
+  int kind = kShotAlone;
+  double drada = 0.0;
 };
 
 // Walk the reference's control flow from the start.  Returns true when the
@@ -1109,6 +1229,8 @@ bool walk(Search& s, int depth, std::vector<double>& want) {
       const auto it = s.table.find(key_of(zinit));
       if (it == s.table.end()) {
         // speculate from here
+        s.kind = bracket ? kShotTree : kShotMarch;
+        s.drada = drada;
         if (!bracket) {
           // the march: zinit, zinit -/+ dzz(zinit), ... while the loop
           // condition would still hold
@@ -1242,7 +1364,7 @@ int ah_record_doubles() { return AF_N; }
 // also its surfaces, trigonometric tables and one search's staging
 double ah_fixed_bytes(int n_ah, int method) {
   double b = static_cast<double>(sizeof(AhCtx)) + 2.0 * n_ah * sizeof(double) * (kAhNthetaMax + 1) +
-             static_cast<double>(kAhScanChunk) * 2.0 * (sizeof(ShotIn) + sizeof(ShotOut));
+             static_cast<double>(kAhScanChunk) * 2.0 * (sizeof(ShotIn) + sizeof(ShotOut) + 2 * sizeof(int));
   if (method != OA_AH_SHOOT)
     b += n_ah * sizeof(double) * (kSpecThetaMax + 1) + 2.0 * sizeof(double) * (kSpecModes + 1) * (kSpecThetaMax + 1) +
          static_cast<double>(n_ah) * (sizeof(SpecIn) + sizeof(SpecOut));
@@ -1262,6 +1384,7 @@ void ah_release(oa_handle* h) {
   }
   if (a->d_in) (void)hipFree(a->d_in);
   if (a->d_out) (void)hipFree(a->d_out);
+  if (a->d_done) (void)hipFree(a->d_done);
   if (a->h_in) (void)hipHostFree(a->h_in);
   if (a->h_out) (void)hipHostFree(a->h_out);
   for (int k = 0; k < 3; ++k)
@@ -1437,14 +1560,17 @@ int run_walks(std::vector<Job>& jobs, hipStream_t st) {
         j.done = true;
         continue;
       }
-      for (double z : want) {
-        in.push_back(ShotIn{j.h->ah->dctx, z, j.s.zcenter, nullptr, nullptr});
+      const int base = static_cast<int>(in.size()), n = static_cast<int>(want.size());
+      for (int at = 0; at < n; ++at) {
+        const double z = want[static_cast<size_t>(at)];
+        in.push_back(ShotIn{j.h->ah->dctx, z, j.s.zcenter, nullptr, nullptr, j.s.kind, base, at, n, j.s.drada});
         owner.push_back({q, z});
       }
     }
     if (in.empty()) break;
     AH_RC(run_shots(st, buf, in, res));
-    for (size_t t = 0; t < in.size(); ++t) jobs[owner[t].first].s.table[key_of(owner[t].second)] = res[t];
+    for (size_t t = 0; t < in.size(); ++t)
+      if (res[t].err != kShotDropped) jobs[owner[t].first].s.table[key_of(owner[t].second)] = res[t];
   }
   for (size_t q = 0; q < jobs.size(); ++q) {
     if (!ran[q]) continue;

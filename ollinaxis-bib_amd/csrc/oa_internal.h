@@ -214,6 +214,9 @@ int launch_norms_partial(const KGrid& G, const double* f, double* part, void* st
 int norms_max_fields();
 int launch_norms_fields_noalloc(int dev, const KGrid& G, int n, const double* const* planes, double* out,
                                 void* stream);
+// one array of a level, ghosts included, to host memory the device can write,
+// rho fastest and (Nr + g) values a row
+int launch_plane_out(const KGrid& G, const double* src, double* host, void* stream);
 int launch_dtbeta_init(const KGrid& G, double csi, bool scalar, double* y, void* stream);
 int launch_fb_table(const KGrid& Gf, const KGrid& Gc, int depth, int interporder, FbPoint* table, long n,
                     void* stream);

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <vector>
 
 #include "oa_internal.h"
@@ -54,8 +55,10 @@ struct oa_handle {
   oa_batch* batch = nullptr;
   oax::KPhys phys{};
   oax::Plan plan;                    // launches of this handle's own calls
-  double* norms_part = nullptr;      // partial records of the 0D norms
   oax::AhState* ah = nullptr;        // horizon finder state (on demand)
+  std::mutex out_lock;               // of host_plane
+  double* host_plane = nullptr;      // pinned: an array or the norms' partials on their way out
+  size_t host_plane_len = 0;
   // timing
   hipEvent_t ev_begin = nullptr, ev_end = nullptr;
   double last_ms = 0.0;

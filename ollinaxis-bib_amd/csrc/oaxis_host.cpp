@@ -441,11 +441,6 @@ extern "C" int oa_create(const oa_params* pin, oa_handle** out) {
     oa_set_error("HIP event creation failed");
     return OA_ERR_HIP;
   }
-  if (hipMalloc(reinterpret_cast<void**>(&h->norms_part), sizeof(double) * 6 * norms_blocks()) != hipSuccess) {
-    oa_destroy(h);
-    oa_set_error("device allocation failed");
-    return OA_ERR_NOMEM;
-  }
   h->L.resize(h->nlev);
   for (int l = 0; l < h->nlev; ++l) {
     Level& L = h->L[l];
@@ -512,9 +507,9 @@ extern "C" int oa_destroy(oa_handle* h) {
   }
   ah_release(h);
   h->plan.release();
-  if (h->norms_part) (void)hipFree(h->norms_part);
   if (h->ev_begin) (void)hipEventDestroy(h->ev_begin);
   if (h->ev_end) (void)hipEventDestroy(h->ev_end);
+  if (h->host_plane) (void)hipHostFree(h->host_plane);
   if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
   delete h;
   return OA_OK;
@@ -565,6 +560,19 @@ extern "C" int oa_upload_field(oa_handle* h, int box, int level, const char* nam
   return OA_OK;
 }
 
+namespace {
+// the handle's pinned plane holds len values; the caller holds out_lock
+int host_plane(oa_handle* h, size_t len) {
+  if (h->host_plane_len >= len) return OA_OK;
+  if (h->host_plane) (void)hipHostFree(h->host_plane);
+  h->host_plane = nullptr;
+  h->host_plane_len = 0;
+  HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&h->host_plane), sizeof(double) * len, hipHostMallocDefault));
+  h->host_plane_len = len;
+  return OA_OK;
+}
+}  // namespace
+
 extern "C" int oa_download_field(oa_handle* h, int box, int level, const char* name, double* dst, int ld) {
   Level* L = level_of(h, box, level);
   if (!L || !name || !dst) return OA_ERR_ARG;
@@ -575,43 +583,59 @@ extern "C" int oa_download_field(oa_handle* h, int box, int level, const char* n
     return OA_ERR_ARG;
   }
   const std::string nm(name);
-  auto fetch = [&](int slot, std::vector<double>& buf) -> int {
-    buf.resize(static_cast<size_t>(G.plane));
-    double* y = L->slab[L->in_step ? L->last_out : L->cur];
-    HIPCHK(hipMemcpyAsync(buf.data(), y + static_cast<long>(slot) * G.plane, sizeof(double) * buf.size(),
-                          hipMemcpyDeviceToHost, h->stream));
+  // one array to the handle's pinned plane, rho fastest
+  const std::lock_guard<std::mutex> hold(h->out_lock);
+  const size_t len = static_cast<size_t>(nrt) * nzt;
+  const double* out = nullptr;
+  auto bring = [&](const double* plane) -> int {
+    RC(host_plane(h, len));
+    RC(launch_plane_out(G, plane, h->host_plane, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    out = h->host_plane;
     return OA_OK;
+  };
+  auto fetch = [&](int slot) -> int {
+    return bring(L->slab[L->in_step ? L->last_out : L->cur] + static_cast<long>(slot) * G.plane);
   };
   auto emit = [&](auto fn) {
     for (int jj = 0; jj < nzt; ++jj)
-      for (int ii = 0; ii < nrt; ++ii) dst[static_cast<size_t>(jj) * ld + ii] = fn(static_cast<size_t>(ii) * G.ld + jj, ii, jj);
+      for (int ii = 0; ii < nrt; ++ii)
+        dst[static_cast<size_t>(jj) * ld + ii] = fn(static_cast<size_t>(jj) * nrt + ii, ii, jj);
+  };
+  auto copy = [&] {
+    if (ld == nrt) std::memcpy(dst, out, sizeof(double) * len);
+    else
+      for (int jj = 0; jj < nzt; ++jj)
+        std::memcpy(dst + static_cast<size_t>(jj) * ld, out + static_cast<size_t>(jj) * nrt, sizeof(double) * nrt);
   };
   const int slot = slot_of(h, nm);
   if (slot >= 0 && !(slot == S_phi && !L->phi_valid)) {
-    std::vector<double> b;
-    RC(fetch(slot, b));
-    emit([&](size_t q, int, int) { return b[q]; });
+    RC(fetch(slot));
+    copy();
     return OA_OK;
   }
   if (nm == "phi" || nm == "psi" || nm == "psi4") {
-    std::vector<double> c;
     if (nm == "phi" || !L->phi_valid) {
-      RC(fetch(S_chi, c));
-      if (nm == "phi") emit([&](size_t q, int, int) { return -0.5 * std::log(c[q]); });
-      else if (nm == "psi") emit([&](size_t q, int, int) { return std::exp(-0.5 * std::log(c[q])); });
-      else emit([&](size_t q, int, int) { return 1.0 / (c[q] * c[q]); });
+      RC(fetch(S_chi));
+      if (nm == "phi") emit([&](size_t q, int, int) { return -0.5 * std::log(out[q]); });
+      else if (nm == "psi") emit([&](size_t q, int, int) { return std::exp(-0.5 * std::log(out[q])); });
+      else emit([&](size_t q, int, int) { return 1.0 / (out[q] * out[q]); });
     } else {
-      RC(fetch(S_phi, c));
-      if (nm == "psi") emit([&](size_t q, int, int) { return std::exp(c[q]); });
-      else emit([&](size_t q, int, int) { const double e = std::exp(c[q]); return e * e * e * e; });
+      RC(fetch(S_phi));
+      if (nm == "psi") emit([&](size_t q, int, int) { return std::exp(out[q]); });
+      else emit([&](size_t q, int, int) { const double e = std::exp(out[q]); return e * e * e * e; });
     }
     return OA_OK;
   }
   if (nm == "KTH" || nm == "lambda" || nm == "Alambda") {
     std::vector<double> A, B, H, C, KA, KB, KC;
-    RC(fetch(S_A, A)); RC(fetch(S_B, B)); RC(fetch(S_H, H)); RC(fetch(S_C, C));
-    RC(fetch(S_KTA, KA)); RC(fetch(S_KTB, KB)); RC(fetch(S_KTC, KC));
+    auto keep = [&](int s, std::vector<double>& v) -> int {
+      RC(fetch(s));
+      v.assign(out, out + len);
+      return OA_OK;
+    };
+    RC(keep(S_A, A)); RC(keep(S_B, B)); RC(keep(S_H, H)); RC(keep(S_C, C));
+    RC(keep(S_KTA, KA)); RC(keep(S_KTB, KB)); RC(keep(S_KTC, KC));
     emit([&](size_t q, int ii, int) {
       const double r = (static_cast<double>(ii + 1 - G.g) - 0.5) * G.dr;
       const double gA = B[q] * H[q], gB = A[q] * H[q], gC = -C[q] * H[q];
@@ -627,11 +651,8 @@ extern "C" int oa_download_field(oa_handle* h, int box, int level, const char* n
       oa_set_error(std::string("oa_download_field: ") + name + " needs oa_constraints on the current state first");
       return OA_ERR_STATE;
     }
-    std::vector<double> b(static_cast<size_t>(G.plane));
-    HIPCHK(hipMemcpyAsync(b.data(), L->cons + static_cast<long>(cons_slot(nm)) * G.plane, sizeof(double) * b.size(),
-                          hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    emit([&](size_t q, int, int) { return b[q]; });
+    RC(bring(L->cons + static_cast<long>(cons_slot(nm)) * G.plane));
+    copy();
     return OA_OK;
   }
   if (nm == "dtalpha" || nm == "dtphi" || nm == "z4theta") {
@@ -687,14 +708,15 @@ extern "C" int oa_norms0d(oa_handle* h, int box, int level, const char* name, do
   if (!L || !name || !out) return OA_ERR_ARG;
   const double* plane = nullptr;
   RC(norms_plane(h, L, "oa_norms0d", name, &plane));
-  RC(launch_norms_partial(L->G, plane, h->norms_part, h->stream));
+  // the blocks' partials are written straight into pinned host memory
   const int nb = norms_blocks();
-  std::vector<double> part(static_cast<size_t>(6 * nb));
-  HIPCHK(hipMemcpyAsync(part.data(), h->norms_part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, h->stream));
+  const std::lock_guard<std::mutex> hold(h->out_lock);
+  RC(host_plane(h, static_cast<size_t>(6 * nb)));
+  RC(launch_norms_partial(L->G, plane, h->host_plane, h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
   double vmax = -1.0e300, vmin = 1.0e300, vabs = 0.0, sq = 0.0, cnt = 0.0, nan = 0.0;
   for (int b = 0; b < nb; ++b) {
-    const double* o = &part[static_cast<size_t>(6 * b)];
+    const double* o = h->host_plane + static_cast<size_t>(6 * b);
     vmax = std::fmax(vmax, o[0]);
     vmin = std::fmin(vmin, o[1]);
     vabs = std::fmax(vabs, o[2]);
@@ -757,7 +779,7 @@ extern "C" int oa_params_footprint(const oa_params* pin, double* bytes) {
   if (!p.eqsym && ((p.Nztotal + p.ghost) % 2 == 0)) p.Nztotal += 1;
   const bool shift = (p.shift != OA_SHIFT_NONE), scalar = (p.mattertype & OA_MATTER_SCALAR) != 0;
   const double nf = nslots(shift, scalar);
-  double total = sizeof(double) * 6.0 * norms_blocks();
+  double total = 0.0;
   for (int l = 0; l <= p.Nl0; ++l) {
     KGrid G;
     fill_grid(G, p, l);

@@ -59,9 +59,9 @@ struct EllCtl {
   int stationary;  // 1: the all-levels phase may end on the stationary rule
   double gres;     // residual of the last step
   double wmax, wprev;   // stationary rule: window maxima of the relative change of u
-  // a level's clock advances at the end of its step (:997-1004).  The last
-  // iteration of the step marks it here, and the next saveold launched (of
-  // any level) applies it: every kernel that reads a level's clock (the
+  // a level's clock advances at the end of its step (:997-1004).  Iteration by
+  // iteration (k_ell_step rotates the clocks itself), the last iteration of the
+  // step marks it here, and the next saveold launched (of any level) applies it: every kernel that reads a level's clock (the
   // iterations and finebounds of that level and of the next finer one)
   // comes after a saveold, and no other kernel reads the clocks.
   int tick[kEllMaxLevels];
@@ -69,9 +69,10 @@ struct EllCtl {
   unsigned arrived;     // blocks of k_ell_check that have written their partials
 };
 
-// One level's planes for the solve.  u, v: the state at the end of a step
-// (also the input of the first iteration); up, vp: the state at the start of
-// the step (saveold); t1/t2: outputs of the intermediate iterations; ua, va:
+// One level's planes for the solve, iteration by iteration (k_ell_step rotates
+// the state through u/v, up/vp and t1u/t1v, and uses no strips).  u, v: the
+// state at the end of a step (also the input of the first iteration); up, vp:
+// the state at the start of the step (saveold); t1/t2: outputs of the intermediate iterations; ua, va:
 // RK4 accumulators; s0, s1, s5: the coefficients; sv: the last source of v
 // (base level, for the residual).  Strips: 3 time levels of the fine-boundary
 // zone for u and v, in the layout of saveold_point (rR, then zL, then zR per

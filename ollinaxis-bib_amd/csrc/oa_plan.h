@@ -121,7 +121,9 @@ struct Plan {
         it.strip0 = strips;
         strips += rhs_strips(it);
         any_pre = any_pre || (it.S.dtb_pre != nullptr);
-        points += static_cast<double>(it.G.Nr) * static_cast<double>(it.G.Nz);
+        // the outer rows as an item of their own (rhs_add_frame) are points of
+        // the level that the item before them counts
+        if (!it.skip) points += static_cast<double>(it.G.Nr) * static_cast<double>(it.G.Nz);
       }
     const size_t off = (arena.size() + kAlign - 1) / kAlign * kAlign;
     arena.resize(off + sizeof(Item) * items.size());

@@ -294,8 +294,7 @@ OA_HD void project(Proj& q, double r, bool time0, int chimethod, bool matter) {
 }
 
 // write v at (i,j) and, inside the symmetry bands, its parity images
-OA_HD void put(double* __restrict__ plane, const KGrid& G, int i, int j, double v,
-                                    double symr, double symz) {
+OA_HD void put(double* plane, const KGrid& G, int i, int j, double v, double symr, double symz) {
   plane[IDX(G, i, j)] = v;
   if (i <= G.g) plane[IDX(G, 1 - i, j)] = symr * v;
   if (G.eqsym && j >= 1 && j <= G.g) {
@@ -329,10 +328,12 @@ OA_HD void slot_parity(bool shift, bool scalar, int s, double& symr, double& sym
 // (k_rhs_phases), and phase 1 alone for the constraints.  The other
 // configurations take rhs_roles (oaxis_rhs.h), which sums the same terms in
 // another order.
+//
+// yout is yp on a step's last substep (neither is __restrict__): y_p is read
+// at the point itself alone, and a thread's reads come before its writes.
 template <bool SHIFT, bool PHIMODE, bool IN, int STAGE, class View>
-OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View& V,
-                     const double* __restrict__ yp, double* __restrict__ acc, double* __restrict__ yout,
-                     double* __restrict__ gaux, int i, int j) {
+OA_HD void rhs_point(const KGrid& G, const KPhys& P, const KStep& S, const View& V, const double* yp,
+                     double* __restrict__ acc, double* yout, double* __restrict__ gaux, int i, int j) {
 
   const long pl = G.plane;
   auto fld = [&](int s) { return V.fld(s); };
@@ -1169,9 +1170,15 @@ constexpr int finebound_groups(bool shift, bool scalar) { return 3 + nslots(shif
 // b0(s): field s at the point at time level t0 (var_p); r1, zL1, zR1: the
 // strips of time level t-1.  Fields are interpolated two at a time, so that
 // their 32 loads are in flight together and no more registers are held.
+//
+// Where finebound rides on a step's last substep, b0 reads the plane yf points
+// to (so yf is not __restrict__).  It is right because a group asks b0 for the
+// fields that it writes and no others, before it writes them, at its own point,
+// and every point has one record: no thread reads what another one writes.  A
+// group that reads one more field would race.
 template <bool SHIFT, bool SCALAR, class B0>
 OA_HD void finebound_point(const KGrid& Gf, const KGrid& Gc, const KPhys& P, const KTime& T, int time0,
-                           const double* __restrict__ yc, double* __restrict__ yf, const double* __restrict__ r1,
+                           const double* __restrict__ yc, double* yf, const double* __restrict__ r1,
                            const double* __restrict__ zL1, const double* __restrict__ zR1, const FbPoint& fp_in,
                            int grp, const B0& b0) {
   const FbPoint fp = fp_in;   // the whole record in one go

@@ -137,9 +137,12 @@ __device__ __forceinline__ void stage_inv_r(const KGrid& G, double* rinv, int ib
 // 64 records of one field group of finebound, or 64 points of one field's
 // strips of saveold.  Finebound reads the coarse level, the step's start at
 // its own points and the strips of time level t-1, and writes only the zone,
-// which the substep leaves alone; saveold reads the step's start.  So both run
-// beside the tiles, and a level step is one launch per substep instead of two
-// and a saveold (each a few us that leave most of the GPU idle).
+// which the substep leaves alone; on the last substep, whose output is the
+// step's start, each of its groups reads only what it overwrites itself
+// (finebound_point).  Saveold rides on the first substep, whose output is never
+// the step's start that it reads.  So both run beside the tiles, and a level
+// step is one launch per substep instead of two and a saveold (each a few us
+// that leave most of the GPU idle).
 __device__ __forceinline__ int edge_fb_units(long n, int groups) { return groups * static_cast<int>((n + 63) / 64); }
 
 template <bool SHIFT, bool SCALAR>

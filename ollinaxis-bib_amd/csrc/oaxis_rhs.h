@@ -118,7 +118,10 @@ enum RhsRole { ROLE_K = 1, ROLE_DELTA = 2, ROLE_LAPSE = 4, ROLE_METRIC = 8, ROLE
 
 // accumulate (prl/arrays.pl:533-599) and update (:1282-1328) of the N slots
 // one part owns; y_p and the accumulators of all of them are loaded together
-// before the first store (one memory round trip; stores would serialise them)
+// before the first store (one memory round trip; stores would serialise them).
+// On a step's last substep the output plane is y_p itself: a part reads y_p of
+// the slots it owns and of no others, at its own point, so the parts of other
+// waves may write theirs in any order.
 template <int N>
 struct RkUpdate {
   double yv[N], av[N];
@@ -228,7 +231,7 @@ OA_HD Matter matter_point(const KPhys& P, const View& V, int i, int j, double r,
 
 template <bool SHIFT, bool SCALAR, bool PHIMODE, bool IN, int ROLE, class View>
 OA_HD void rhs_roles(const KGrid& G, const KPhys& P, const KStep& S, const KStencil& W, const View& V,
-                     const double* __restrict__ yp, double* __restrict__ acc, double* __restrict__ yout, int i, int j) {
+                     const double* yp, double* __restrict__ acc, double* yout, int i, int j) {
 
   const long pl = G.plane;
   auto fld = [&](int s) { return V.fld(s); };

@@ -53,6 +53,7 @@
 #define OA_HD __device__ __forceinline__
 #define OA_HHD __host__ __device__ inline
 #include "oaxis_device.h"
+#include "oaxis_recip.h"
 
 namespace oax {
 namespace {
@@ -273,34 +274,6 @@ struct AhCell {
 // near the level's edges (or with interporder = bilinear), else bicubic
 // Lagrange weights.  Formed once per point; ah_combine applies it to the
 // records of one quantity with the reference's expressions.
-//
-// Quotients by one divisor share its reciprocal: two Newton steps on the
-// hardware's estimate, then per quotient a product and one residual correction
-// (Markstein 1990), which rounds correctly wherever numerator, divisor and
-// quotient are normal numbers; three instructions instead of eleven.  A
-// division by zero or of an infinity gives NaN, which the sources refuse as
-// they refuse an infinity.
-struct AhRecip {
-  double d, y;
-  __device__ __forceinline__ explicit AhRecip(double div) : d(div) {
-    y = __builtin_amdgcn_rcp(d);
-    y = fma(y, fma(-d, y, 1.0), y);
-    y = fma(y, fma(-d, y, 1.0), y);
-  }
-  __device__ __forceinline__ AhRecip(double div, double recip) : d(div), y(recip) {}
-  __device__ __forceinline__ double of(double x) const {
-    const double q = x * y;
-    return fma(fma(-d, q, x), y, q);
-  }
-};
-
-// x / n for the bicubic weights' n, 1 <= |n| <= 3
-__device__ __forceinline__ double ah_over(double x, int n) {
-  const int m = n < 0 ? -n : n;
-  const double q = (m == 3) ? AhRecip(3.0, 1.0 / 3.0).of(x) : (m == 2) ? 0.5 * x : x;
-  return n < 0 ? -q : q;
-}
-
 struct AhPlan {
   int lev, i0, j0, mode;              // mode 0: node copy, 1: bilinear, 2: bicubic
   double auxr, auxz;

@@ -1,8 +1,11 @@
 """GPU: the relaxation's level steps at the edges of their tiles (elliptic.hip;
 wave_elliptic.f90:542-1164), against the oracle's solve with the same number
-of steps.  A level step of the default relaxation runs by tiles of 16 x 16
-points, so the grids end one point before, on and after a tile; RK4 goes
-iteration by iteration, here with a fine level's boundary.  Bound: the steps
+of steps.  A level step of the default relaxation runs by tiles of 8 x 16
+points along rho and z, and by tiles of 16 x 16 where those number 256 or more
+(256 x 256 points and up): the grids end one point before, on and after a tile
+of each form, with and without equatorial symmetry, a fine boundary and the
+u^5 term, and 240 x 271 (255 tiles) is the last size of the smaller one.  RK4
+goes iteration by iteration, here with a fine level's boundary.  Bound: the steps
 are the same sums in another order, rounded at 2^-53 each; a step has under
 2^7 of them and the damped relaxation does not amplify, so 120 coarse steps
 (with subcycling under 2^9 level steps) stay within 2^-53 * 2^16 < 1e-10 of
@@ -22,6 +25,12 @@ CASES = {
     "whole_plane_18x45": (PULSE, 18, 45, 1, "eqsym = .false.\n"),
     "potential_33x16": (PULSE, 33, 16, 2, "eqsym = .true.\nscalarpotential = phi2\nscalar_mass = 0.1\n"),
     "brill_49x31": (BRILL, 49, 31, 0, ""),
+    "last_of_8_rows_240x271": (PULSE, 240, 271, 0, "eqsym = .true.\n"),
+    "rows_16_tiles_256x271": (PULSE, 256, 271, 0, "eqsym = .true.\n"),
+    "rows_16_one_past_257x273": (PULSE, 257, 273, 0, "eqsym = .true.\n"),
+    "rows_16_one_before_271x271": (BRILL, 271, 271, 0, ""),
+    "rows_16_fine_259x256": (PULSE, 259, 256, 1, "eqsym = .false.\n"),
+    "rows_16_potential_257x272": (PULSE, 257, 272, 1, "eqsym = .true.\nscalarpotential = phi2\nscalar_mass = 0.1\n"),
     "rk4_18x34": (PULSE, 18, 34, 1, "eqsym = .false.\nWE_method = rk4\n"),
 }
 

@@ -29,10 +29,10 @@
 //     continuation at once: during the march, the next positions down the
 //     axis; during the bisection, the full tree of the next bisection steps,
 //     as deep as gives every shot of every search a SIMD of its own
-//     (kAhResident waves in all, at most kAhMaxDepth steps).  The walk then
-//     takes exactly the reference's path through those results, so the
-//     sequence of shots and every decision are the reference's; shots that
-//     finished ones exclude end early, and unused ones are discarded.
+//     (kAhResident waves in all).  The walk then takes exactly the
+//     reference's path through those results, so the sequence of shots and
+//     every decision are the reference's; shots that finished ones exclude
+//     end early, and unused ones are discarded.
 //
 // Floating-point contraction is off in this file, so the sources and the
 // interpolation round like the oracle's IEEE build of the same expressions.
@@ -54,6 +54,7 @@
 #define OA_HHD __host__ __device__ inline
 #include "oaxis_device.h"
 #include "oaxis_recip.h"
+#include "oaxis_shots.h"
 
 namespace oax {
 namespace {
@@ -65,12 +66,13 @@ constexpr int kAhNthetaMax = 50000;                 // Nthetamax (:350)
 // bound is reached only by a shot the reference would integrate for hours.
 constexpr int kAhMaxSteps = 4 * kAhNthetaMax;
 constexpr int kAhScanChunk = 1024;                  // march positions per launch
-constexpr int kAhMaxDepth = 11;                     // bisection steps per launch, at most
-// Shots of one launch: one wave to a SIMD (256 CUs x 4).  A shot is bound by
-// the issue of its own serial chain, so two waves on a SIMD take twice as long
-// (a tree of 11 steps 12.0 ms where one shot alone took 6.0), for one
-// bisection step more.
+constexpr int kAhMaxDepth = 10;                     // bisection steps per launch, at most
+// Shots of one launch: one wave to a SIMD (256 CUs x 4): the 1023
+// nodes of a tree of kAhMaxDepth steps.  A shot is bound by the issue of its own
+// serial chain, so two waves on a SIMD take twice as long (a tree of 11 steps
+// 12.0 ms where one shot alone took 6.0), for one bisection step more.
 constexpr int kAhResident = 1024;
+static_assert((1 << kAhMaxDepth) - 1 <= kAhResident, "one search's deepest tree has a SIMD per shot");
 constexpr int kShotBlock = 64;
 
 // interpolated quantities, in ah_source's order
@@ -111,13 +113,9 @@ struct ShotOut {
 };
 constexpr int kShotDropped = -1;      // ShotOut::err: not integrated to its end
 
-// Speculative shots that can no longer be asked for end early (two levels of
-// 128 x 256: the march's launch 21.5 -> 18.1 ms, the first tree's 25.9 -> 18.4
-// together with its smaller depth).  A march ends
-// at the first pair of neighbours whose end slopes differ in sign, so the
-// shots past a finished such pair are dropped; a node of the bisection's tree
-// sends the walk into one of its two subtrees, so a finished node drops the
-// other.  Only shots whose need is excluded by finished ones are dropped, and
+// Speculative shots that can no longer be asked for (oaxis_shots.h) end early
+// (two levels of 128 x 256: the march's launch 21.5 -> 17.7 ms, the first tree's
+// 25.9 -> 18.4 together with its smaller depth).  Only shots whose need is excluded by finished ones are dropped, and
 // the first shot of a launch never is, so each launch brings the walk on; a
 // dropped shot that is asked for later all the same is launched again.  Each
 // shot looks once per step, with a load that the step's sources hide; nothing
@@ -136,7 +134,7 @@ __device__ __forceinline__ int shot_look(const ShotIn& s, const int* done, int t
   const int lane = static_cast<int>(threadIdx.x);
   if (s.kind == kShotMarch) return lane == 0 ? shot_word(done, total + s.base) : 0;
   if (s.kind != kShotTree || lane >= kAhMaxDepth) return 0;
-  const int up = (s.at + 1) >> (lane + 1);
+  const int up = tree_number(s.at, lane + 1);
   return up > 0 ? shot_word(done, s.base + up - 1) : 0;
 }
 
@@ -144,10 +142,9 @@ __device__ __forceinline__ bool shot_dropped(const ShotIn& s, int word) {
   const int lane = static_cast<int>(threadIdx.x);
   bool drop = false;
   if (s.kind == kShotMarch) {
-    drop = lane == 0 && word > 0 && s.at > s.n - word;
+    drop = lane == 0 && march_excluded(s.at, s.n, word);
   } else if (s.kind == kShotTree) {
-    const bool right = (((s.at + 1) >> lane) & 1) != 0;    // the child of that ancestor the shot is below
-    drop = lane < kAhMaxDepth && (word & (right ? 2 : 1)) != 0;
+    drop = lane < kAhMaxDepth && tree_excluded(s.at, lane + 1, word);
   }
   return __any(drop);
 }
@@ -156,8 +153,8 @@ __device__ __forceinline__ bool shot_dropped(const ShotIn& s, int word) {
 __device__ __forceinline__ void shot_publish(const ShotIn& s, int* done, int total, const ShotOut* out, double d) {
   if (s.kind == kShotTree) {
     const double p = s.drada * d;
-    if (p <= 0.0) atomicOr(done + s.base + s.at, 2);
-    else if (p > 0.0) atomicOr(done + s.base + s.at, 1);
+    if (excludes_right(p)) atomicOr(done + s.base + s.at, 2);
+    else if (excludes_left(p)) atomicOr(done + s.base + s.at, 1);
   } else if (s.kind == kShotMarch) {
     __threadfence();
     atomicOr(done + s.base + s.at, 1);
@@ -166,7 +163,7 @@ __device__ __forceinline__ void shot_publish(const ShotIn& s, int* done, int tot
       __threadfence();
       const double o = __hip_atomic_load(&out[s.base + q].dradlast, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int end = s.at > q ? s.at : q;
-      if (!(d * o >= 0.0)) atomicMax(done + total + s.base, s.n - end);
+      if (march_ends(d, o)) atomicMax(done + total + s.base, s.n - end);
     }
   }
 }

@@ -72,6 +72,14 @@ OA_HD D2 hess(const F& f, const KGrid& G, const KStencil& W, int i, int j) {
 // sides cost one expression, without a branch or a select.  With centred
 // advection (shiftadvect = .false.) the weights are those of the centred
 // derivative; the scalar field is upwinded always (ADV = 2).
+//
+// The weights of this sum are larger than the upwind stencil's (60/12 of f/h
+// against 38/12), and summed over the values f themselves it rounds up to 1.6
+// times as far off.  So it is summed over the differences f(k) - f(0), which
+// are exact, or nearly so, wherever the grid resolves f: the error is then 0.01
+// to 0.25 of the stencil's on fields near one and 0.7 to 0.9 of it on fields near
+// zero.  The differences replace the values in registers; the 12 additions more
+// cost a batch of 16 pulses 69.5 -> 70.6 ms, less than its runs differ by.
 template <bool IN, int ADV, class F>
 OA_HD double advdis(const F& f, const KGrid& G, const KPhys& P, const KStencil& W, int i, int j, double br, double bz,
                     double ko, bool dis) {
@@ -81,18 +89,23 @@ OA_HD double advdis(const F& f, const KGrid& G, const KPhys& P, const KStencil& 
     const double rp3 = f(i + 3, j), rm3 = f(i - 3, j);
     const double zp = f(i, j + 1), zm = f(i, j - 1), zp2 = f(i, j + 2), zm2 = f(i, j - 2);
     const double zp3 = f(i, j + 3), zm3 = f(i, j - 3);
-    const double d6r = 20.0 * c - 15.0 * (rp + rm) + 6.0 * (rp2 + rm2) - (rp3 + rm3);
-    const double d6z = 20.0 * c - 15.0 * (zp + zm) + 6.0 * (zp2 + zm2) - (zp3 + zm3);
-    if constexpr (ADV == 2) {
-      const double odr = W.r12 * (10.5 * (rp - rm) - 3.0 * (rp2 - rm2) + 0.5 * (rp3 - rm3));
-      const double odz = W.z12 * (10.5 * (zp - zm) - 3.0 * (zp2 - zm2) + 0.5 * (zp3 - zm3));
-      return br * odr + bz * odz - (ko + 0.5 * W.r12 * fabs(br)) * d6r - (ko + 0.5 * W.z12 * fabs(bz)) * d6z;
-    } else if constexpr (ADV == 1) {
-      const double odr = W.ar[0] * (rp - rm) + W.ar[1] * (rp2 - rm2) + W.ar[2] * (rp3 - rm3);
-      const double odz = W.az[0] * (zp - zm) + W.az[1] * (zp2 - zm2) + W.az[2] * (zp3 - zm3);
-      return br * odr + bz * odz - (ko + W.ur * fabs(br)) * d6r - (ko + W.uz * fabs(bz)) * d6z;
-    } else {
+    if constexpr (ADV == 0) {
+      const double d6r = 20.0 * c - 15.0 * (rp + rm) + 6.0 * (rp2 + rm2) - (rp3 + rm3);
+      const double d6z = 20.0 * c - 15.0 * (zp + zm) + 6.0 * (zp2 + zm2) - (zp3 + zm3);
       return -ko * (d6r + d6z);
+    }
+    const double ap = rp - c, am = rm - c, ap2 = rp2 - c, am2 = rm2 - c, ap3 = rp3 - c, am3 = rm3 - c;
+    const double bp = zp - c, bm = zm - c, bp2 = zp2 - c, bm2 = zm2 - c, bp3 = zp3 - c, bm3 = zm3 - c;
+    const double d6r = 6.0 * (ap2 + am2) - 15.0 * (ap + am) - (ap3 + am3);
+    const double d6z = 6.0 * (bp2 + bm2) - 15.0 * (bp + bm) - (bp3 + bm3);
+    if constexpr (ADV == 2) {
+      const double odr = W.r12 * (10.5 * (ap - am) - 3.0 * (ap2 - am2) + 0.5 * (ap3 - am3));
+      const double odz = W.z12 * (10.5 * (bp - bm) - 3.0 * (bp2 - bm2) + 0.5 * (bp3 - bm3));
+      return br * odr + bz * odz - (ko + 0.5 * W.r12 * fabs(br)) * d6r - (ko + 0.5 * W.z12 * fabs(bz)) * d6z;
+    } else {
+      const double odr = W.ar[0] * (ap - am) + W.ar[1] * (ap2 - am2) + W.ar[2] * (ap3 - am3);
+      const double odz = W.az[0] * (bp - bm) + W.az[1] * (bp2 - bm2) + W.az[2] * (bp3 - bm3);
+      return br * odr + bz * odz - (ko + W.ur * fabs(br)) * d6r - (ko + W.uz * fabs(bz)) * d6z;
     }
   } else {
     double s = 0.0;

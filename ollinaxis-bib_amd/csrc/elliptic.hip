@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(kBlk) k_ell_iter_fb(EllStepArgs a, EllCtl* ctl
 // the third.  The level's clock rotates with them.
 // Tiles of 8 x 16 points where 16 x 16 would leave compute units without a
 // block: half as much again per point, but shorter chains and twice the blocks
-// (128 x 256 with equatorial symmetry: 128 blocks 11.0 us, 256 blocks 9.8).
+// (128 x 256 with equatorial symmetry: 128 blocks 11.0 us, 256 blocks 9.9).
 constexpr int kEsTile = 16, kEsHalo = 9, kEsW = kEsTile + 2 * kEsHalo;
 constexpr int kEsFill = 256;       // blocks that give every compute unit one
 
@@ -656,7 +656,7 @@ __global__ void __launch_bounds__(kBlk) k_ell_restrict(EllRsArgs a, const EllCtl
 // Bound by latency (the launch, two round trips, the arrivals at one counter
 // and the partials' way between the dies): few blocks, one point a thread up
 // to 128 x 256, reductions in registers.  256 blocks with trees in LDS and a
-// serial sum took 11.4 us of a step of 128 x 256, this 5.2.
+// serial sum took 11.4 us of a step of 128 x 256, this 5.7.
 struct EllCheckArgs {
   KGrid G;
   const double *sv, *u, *up;

@@ -81,8 +81,8 @@ namespace oax {
 int niter_of(const oa_handle* h);
 void substep_weights(const oa_handle* h, int level, int iter, double* dtw, double* w);
 int prepare_saveold(oa_handle* h, int level, SaveItem* it);
-// *inner: the item leaves out the outer rows that finebound fills (rhs_frame
-// gives them)
+// *inner: the item leaves out the outer rows that finebound fills
+// (rhs_add_frame gives them)
 int prepare_substep(oa_handle* h, int level, int iter, int niter, double dtw, double w, RhsItem* it,
                     bool* phimode, bool* inner);
 bool prepare_finebound(oa_handle* h, int level, double dtw, FbItem* it);   // false on level 0

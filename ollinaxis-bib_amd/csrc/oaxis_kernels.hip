@@ -304,8 +304,9 @@ __device__ __forceinline__ int xcd_block(int b, int total) {
 // a tile inside: they start first and are spread over the XCDs.  Four waves on a
 // SIMD hide the stencils' LDS latency, which bounded the sources in two phases
 // of four waves: 512 x 1024 in vacuum 80.4 -> 55 us a launch (its bytes take 44
-// at the rate of a large copy), 128 x 256 with Gamma-driver and scalar field 19.9
-// us with its finebound and saveold, which were launches of their own.
+// at the rate of a large copy); a fine level of 128 x 256 with Gamma-driver and
+// scalar field 17 us with its finebound, 20 with its saveold too, which were
+// launches of their own.
 template <bool SHIFT, bool SCALAR, bool PHIMODE>
 __global__ void __launch_bounds__(kRhsBlock, 4) k_rhs_table(const RhsItem* __restrict__ items, int n, int strips,
                                                             int xcd_remap) {
@@ -363,17 +364,6 @@ __device__ __forceinline__ void stage_planes(double* tile, int first, const Phas
   }
 }
 
-// The Gamma-driver in vacuum: one thread per point in two phases.  Phase 1
-// forms the geometric auxiliaries (the Ricci tensor and div KT: the longest
-// expressions, which need only the vacuum fields) and passes them through the
-// per-level buffer gaux; phase 2 forms D_i D_j alpha, every source, the
-// dissipation, the radiative boundaries and the RK update.  Kept apart, the
-// phases need at most the registers of the larger one: 250 VGPRs, two waves
-// per SIMD, and the staged tile (17 fields, 66 KB) allows two blocks per CU.
-// The roles' kernel is faster here too (a Brill step on 5 levels of 256x512
-// at 4.5 ms with it), but it rounds differently, and the constraints of such
-// data, residuals that amplify the last bit of the state by 1/h^2, then move
-// by up to 3e-9 of their size: this configuration keeps its bits.
 // Whether the point lies in an interior tile of the level's whole tile grid.
 // The two forms of phase 1 contract their sums differently, so a point keeps
 // one form whichever range of the level an item computes.
@@ -383,6 +373,18 @@ __device__ __forceinline__ bool interior_point(const KGrid& G, int i, int j) {
   return interior_tile(G, tile_start(bi, nbi, 1, G.Nr), tile_start(bj, nbj, G.jlo, G.Nz));
 }
 
+// The Gamma-driver in vacuum: one thread per point in two phases.  Phase 1
+// forms the geometric auxiliaries (the Ricci tensor and div KT: the longest
+// expressions, which need only the vacuum fields) and passes them through the
+// per-level buffer gaux; phase 2 forms D_i D_j alpha, every source, the
+// dissipation, the radiative boundaries and the RK update.  Kept apart, the
+// phases need at most the registers of the larger one: 242 VGPRs, two waves
+// per SIMD, and the staged tile (17 fields, 66 KB) allows two blocks per CU.
+//
+// The form by parts would be faster here too, and nothing shows it less accurate.
+// But other sums have other last bits, and the constraints of such data, residuals
+// that amplify the last bit of the state by 1/h^2, move with them by 1e-10 to 3e-9
+// of their size.  That this configuration keeps its bits is a choice.
 template <bool PHIMODE>
 __device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int t, double* tile) {
   constexpr int nf = nslots(true, false);
@@ -430,10 +432,9 @@ __device__ __forceinline__ void rhs_phases_tile(const RhsItem& it, int t, double
   edge_share<true, false>(it, nt, t, wave, kTile * kTile / 64);
 }
 
-// The Gamma-driver in vacuum: 250 VGPRs, two waves on a SIMD, bound by the latency
-// of its LDS reads.  A level of 256 x 512 with its finebound and saveold takes 39
-// us, 61 as launches of their own over all rows.  The form by parts is faster but
-// rounds otherwise, which a Brill wave's constraints show (1e-10 to 3e-9).
+// Two waves on a SIMD, bound by the latency of its LDS reads (half of a wave's
+// life is waits).  A level of 256 x 512 with its finebound and saveold takes 39
+// us; over all rows, without them, it took 62.
 template <bool PHIMODE>
 __global__ void __launch_bounds__(kTile * kTile, 2) k_rhs_phases(const RhsItem* __restrict__ items, int n,
                                                                  int xcd_remap) {
@@ -1066,7 +1067,6 @@ int launch_constraints(const KGrid& G, const KPhys& P, const KStep& S, bool phim
   it.P = P;
   bool inner = false;
   RC_K(rhs_tiles(&it, false, &inner));
-  rhs_stencil(G, P, &it.W);
   it.S = S;
   it.S.dtb_pre = nullptr;
   it.yin = y;

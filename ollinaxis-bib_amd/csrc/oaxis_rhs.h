@@ -125,8 +125,7 @@ OA_HD double advdis(const F& f, const KGrid& G, const KPhys& P, const KStencil& 
 // shift); the lapse and the conformal metric, which the projection couples;
 // and the scalar field.  Each call forms the sources of its own fields, their
 // dissipation, radiative boundaries, RK update and parity images; what a part
-// does not use compiles out.  ROLE_AUX writes the Ricci scalar and div KT of
-// the state to gaux for the constraints instead.
+// does not use compiles out.
 enum RhsRole { ROLE_K = 1, ROLE_DELTA = 2, ROLE_LAPSE = 4, ROLE_METRIC = 8, ROLE_SCALAR = 16 };
 
 // accumulate (prl/arrays.pl:533-599) and update (:1282-1328) of the N slots
@@ -209,25 +208,20 @@ OA_HD D1 grad_phi(const View& V, const KGrid& G, const KStencil& W, int i, int j
 
 // matter terms of the real scalar field (auxiliary_matter / stressenergy)
 struct Matter {
-  double rho, J_r, J_z, S_A, S_B, S_C, trS, VP;
+  double rho, J_r, J_z, S_A, S_B, S_C, trS;
 };
 
-template <bool SHIFT, bool IN, int ROLE, class View>
+template <bool SHIFT, class View>
 OA_HD Matter matter_point(const KPhys& P, const View& V, int i, int j, double r, double ir, double A, double B,
                           double H, double C, double gA, double gB, double gH, double gC, double ipsi4, double psi4) {
   Matter m;
   const double xr = V.fld(scalar_slot(SHIFT, SC_xi_r))(i, j), xz = V.fld(scalar_slot(SHIFT, SC_xi_z))(i, j);
   const double pi = V.fld(scalar_slot(SHIFT, SC_pi))(i, j);
   double Vpot = 0.0;
-  m.VP = 0.0;
   if (P.scalarpotential != OA_POT_NONE) {
     const double ph = V.fld(scalar_slot(SHIFT, SC_phi))(i, j);
     Vpot = 0.5 * P.scalar_mass * P.scalar_mass * ph * ph;
-    m.VP = P.scalar_mass * P.scalar_mass * ph;
-    if (P.scalarpotential == OA_POT_PHI4) {
-      Vpot += 0.25 * P.scalar_lambda * ph * ph * ph * ph;
-      m.VP += P.scalar_lambda * ph * ph * ph;
-    }
+    if (P.scalarpotential == OA_POT_PHI4) Vpot += 0.25 * P.scalar_lambda * ph * ph * ph * ph;
   }
   const double q2 = (gA * xr * xr + gB * xz * xz + 2.0 * r * gC * xr * xz) * ipsi4;
   m.rho = 0.5 * (pi * pi + q2) + Vpot;
@@ -441,7 +435,7 @@ OA_HD void rhs_roles(const KGrid& G, const KPhys& P, const KStep& S, const KSten
         sKC += alpha * (trK * KTC - 2.0 * KT2_C);
       }
       if constexpr (SCALAR) {
-        const Matter m = matter_point<SHIFT, IN, ROLE>(P, V, i, j, r, ir, A, B, H, C, gA, gB, gH, gC, ipsi4, ic * ic);
+        const Matter m = matter_point<SHIFT>(P, V, i, j, r, ir, A, B, H, C, gA, gB, gH, gC, ipsi4, ic * ic);
         strK += 4.0 * smallpi * alpha * (m.rho + m.trS);
         sKA -= 8.0 * smallpi * alpha * (m.S_A * ipsi4 - third * A * m.trS);
         sKB -= 8.0 * smallpi * alpha * (m.S_B * ipsi4 - third * B * m.trS);
@@ -571,7 +565,7 @@ OA_HD void rhs_roles(const KGrid& G, const KPhys& P, const KStep& S, const KSten
       }
       if constexpr (SCALAR) {
         const double psi4 = ic * ic;
-        const Matter m = matter_point<SHIFT, IN, ROLE>(P, V, i, j, r, ir, A, B, H, C, gA, gB, gH, gC, ipsi4, psi4);
+        const Matter m = matter_point<SHIFT>(P, V, i, j, r, ir, A, B, H, C, gA, gB, gH, gC, ipsi4, psi4);
         sDr -= 8.0 * smallpi * eta * alpha * m.J_r * psi4;
         sDz -= 8.0 * smallpi * eta * alpha * m.J_z * psi4;
       }

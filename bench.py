@@ -15,8 +15,10 @@ Prints one JSON line.  Only one GPU is supported: --gpus above 1 exits with
 a message.
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -52,21 +54,54 @@ def bytes_per_update(params, nfields):
     return 8.0 * nfields * (2 + 3 * (it - 1)), it
 
 
+RHS_SOURCES = ("oaxis_device.h", "oaxis_rhs.h", "oaxis_kernels.hip")
+
+
+def code_id(texts):
+    """Sixteen hex digits that change with the code of the given C++ texts and
+    not with their comments, blanks or line breaks."""
+    h = hashlib.sha256()
+    for text in texts:
+        text = re.sub(r"/\*.*?\*/", " ", text, flags=re.S)
+        text = re.sub(r"//[^\n]*", " ", text)
+        h.update(" ".join(text.split()).encode() + b"\0")
+    return h.hexdigest()[:16]
+
+
+def rhs_code():
+    """code_id of the right-hand-side kernels' sources."""
+    texts = []
+    for name in RHS_SOURCES:
+        with open(os.path.join(ROOT, "ollinaxis-bib_amd", "csrc", name)) as f:
+            texts.append(f.read())
+    return code_id(texts)
+
+
+def counter_summary(name, key, workload):
+    """The number on the line `key workload number` of a committed counter
+    summary; None if it has no such line or was taken on other kernels than
+    the present ones (its line `rhs_code id`)."""
+    value, code = None, None
+    try:
+        with open(os.path.join(ROOT, "profiles", name)) as f:
+            for line in f:
+                parts = line.split()
+                if len(parts) == 3 and parts[0] == key and parts[1] == workload:
+                    value = float(parts[2])
+                elif len(parts) == 2 and parts[0] == "rhs_code":
+                    code = parts[1]
+    except OSError:
+        return None
+    return value if code == rhs_code() else None
+
+
 def measured_traffic(workload, algorithmic_bytes):
     """HBM bytes per RHS launch for this workload: the copy-calibrated
     FETCH_SIZE + WRITE_SIZE per point measured for it (committed summary),
     relative to its algorithmic bytes, times the launch's algorithmic bytes;
-    None when no measurement is committed."""
-    path = os.path.join(ROOT, "profiles", "k_rhs_hbm_traffic.md")
-    try:
-        with open(path) as f:
-            for line in f:
-                parts = line.split()
-                if len(parts) == 3 and parts[0] == "traffic_ratio" and parts[1] == workload:
-                    return float(parts[2]) * algorithmic_bytes
-    except OSError:
-        pass
-    return None
+    None when no measurement of the present kernels is committed."""
+    ratio = counter_summary("k_rhs_hbm_traffic.md", "traffic_ratio", workload)
+    return None if ratio is None else ratio * algorithmic_bytes
 
 
 def fp64_roofline(workload, points_per_launch, avg_launch_ms):
@@ -74,17 +109,8 @@ def fp64_roofline(workload, points_per_launch, avg_launch_ms):
     point of one RHS evaluation for this workload (committed summary,
     SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64) times the points one launch
     evaluates, over the launch's average duration; None without a
-    measurement."""
-    path = os.path.join(ROOT, "profiles", "k_rhs_fp64_valu.md")
-    per_point = None
-    try:
-        with open(path) as f:
-            for line in f:
-                parts = line.split()
-                if len(parts) == 3 and parts[0] == "flop_per_point" and parts[1] == workload:
-                    per_point = float(parts[2])
-    except OSError:
-        pass
+    measurement of the present kernels."""
+    per_point = counter_summary("k_rhs_fp64_valu.md", "flop_per_point", workload)
     if per_point is None or avg_launch_ms <= 0.0:
         return None
     tflops = per_point * points_per_launch / (avg_launch_ms * 1e-3) / 1e12
@@ -638,7 +664,8 @@ def main():
                    "point_updates": updates, "device_ms": device_ms, "schedule": schedule},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(args.workload, bytes_per_launch),
-                     "kernel": "k_rhs_table", "avg_launch_ms": rhs_ms, "launches": rhs_n,
+                     "kernel": "k_rhs_phases" if shift and not scalar else "k_rhs_table",
+                     "avg_launch_ms": rhs_ms, "launches": rhs_n,
                      "algorithmic_bytes_per_launch": bytes_per_launch},
         "fp64": fp64_roofline(args.workload, points_per_launch, rhs_ms),
     }

@@ -4,7 +4,9 @@ profiles/k_rhs_fp64_valu.md).  Every workload the bench measures has its
 entries there, and the ratio the bench reads is the one the summary's table
 derives from its measured bytes (read + write per point over the
 algorithmic bytes per point), so that an edit of a summary cannot leave the
-bench reporting a figure the table does not hold."""
+bench reporting a figure the table does not hold.  A summary names the code it
+was taken on, and counters of other kernels than the present ones are left
+out of the line."""
 import os
 import sys
 
@@ -46,3 +48,21 @@ def test_fp64_rates_come_from_the_counter_summary():
         assert abs(f["achieved"] - f["flop_per_point"] * 1.0e6 / 1.0e-3 / 1.0e12) < 1e-9
         assert abs(f["frac"] - f["achieved"] / f["peak"]) < 1e-15
     assert bench.fp64_roofline("batched_scalar", 1.0e6, 0.0) is None
+
+
+def test_counters_of_other_kernels_are_left_out(monkeypatch):
+    import bench
+    monkeypatch.setattr(bench, "rhs_code", lambda: "0" * 16)
+    for w in WORKLOADS:
+        assert bench.measured_traffic(w, 1.0e6) is None
+        assert bench.fp64_roofline(w, 1.0e6, 1.0) is None
+
+
+def test_code_id_follows_the_code_alone():
+    import bench
+    text = "double f(double x) {  // the square\n  return x * x;  /* twice\n x */\n}\n"
+    same = "double f(double x)\n{ // its square\n return x * x; }"
+    assert bench.code_id([text]) == bench.code_id(["double f(double x) { return x * x; }"])
+    assert bench.code_id([text]) == bench.code_id([same])
+    assert bench.code_id([text]) != bench.code_id([text.replace("x * x", "x + x")])
+    assert bench.code_id(["a", "b"]) != bench.code_id(["ab", ""])

@@ -706,7 +706,7 @@ __global__ void __launch_bounds__(256) k_fb_table(KGrid Gf, KGrid Gc, int D, int
                                                   FbPoint* __restrict__ table) {
   const long q = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (q >= n) return;
-  FbPoint fp;
+  FbPoint fp{};               // a record of no point holds zeros: its i and j are read before its kind is looked at
   fb_geometry(Gf, Gc, D, interporder, q, fp);
   table[q] = fp;
 }
